@@ -354,13 +354,6 @@ __device__ __forceinline__ void store_frags_f16_exp(char *base, int off, int idx
 }
 
 
-// Workgroup barrier for LDS hand-offs only: waits for this wave's LDS
-// accesses, not for its outstanding global loads (a full __syncthreads() also
-// drains vmcnt, which would stall the scan's prefetch of the next chunk).
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
 __device__ __forceinline__ void seq_bounds(const KdaChunkArgs &a, int n, int &bos, int &eos) {
     const int T = a.num_tokens;
     bos = a.cu_seqlens[n];

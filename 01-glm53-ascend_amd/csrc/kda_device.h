@@ -101,6 +101,13 @@ __device__ __forceinline__ float dot4(float4 a, float4 b) {
     return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
 }
 
+// Workgroup barrier for LDS hand-offs only: waits for this wave's LDS
+// accesses, not for its outstanding global loads (a full __syncthreads() also
+// drains vmcnt, which would stall prefetches and stores that nothing waits for).
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 
 }  // namespace kda

@@ -23,13 +23,12 @@
 // ds_swizzle when L = 32), so the state tile lives in VGPRs from the first
 // load to the single in-place write-back: HBM sees each state byte exactly
 // once in and once out. A workgroup (4 waves) covers 4*(64/L)*NP value rows
-// of one (sequence, head). The host picks the shape from the tokens per
-// sequence: one or two tokens (decode, short verify) use 32-lane rows, one
-// token with few rows per lane, so the launch has many small workgroups to
-// stream the state; three or more (verify, prefill) use 16-lane rows, whose
-// reductions take four DPP steps instead of five plus an LDS swizzle, with
-// up to eight rows per lane to share each token's loads, exponentials and
-// norms.
+// of one (sequence, head). The host picks the kernel and shape from the
+// tokens per sequence: one token (decode) uses 32-lane rows with few rows per
+// lane, so the launch has many small workgroups to stream the state; more
+// (verify, prefill) run in blocks of tokens prepared once per workgroup, on
+// 16-lane rows, whose reductions take four DPP steps instead of five plus an
+// LDS swizzle.
 
 #include <hip/hip_runtime.h>
 
@@ -102,6 +101,17 @@ template <int NP, int RS> struct RowIn<uint16_t, NP, RS> {
             }
         }
     }
+    // the same from an address of any alignment
+    __device__ __forceinline__ void load_each(const uint16_t *p) {
+        if constexpr (RS != 1) {
+            load(p);
+        } else {
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                w[i] = static_cast<uint32_t>(p[2 * i]) | (static_cast<uint32_t>(p[2 * i + 1]) << 16);
+            }
+        }
+    }
     __device__ __forceinline__ float get(int i) const {
         if constexpr (RS != 1) {
             return __uint_as_float(w[i] << 16);
@@ -111,7 +121,7 @@ template <int NP, int RS> struct RowIn<uint16_t, NP, RS> {
     }
 };
 template <int NP, int RS> struct RowIn<float, NP, RS> {
-    static_assert(RS != 1 || NP % 4 == 0, "whole float4 vectors");
+    static_assert(RS != 1 || NP % 4 == 0 || NP == 2, "whole vectors");
     float x[NP];
     __device__ __forceinline__ void load(const float *p) {
         if constexpr (RS != 1) {
@@ -119,6 +129,10 @@ template <int NP, int RS> struct RowIn<float, NP, RS> {
             for (int i = 0; i < NP; ++i) {
                 x[i] = p[RS * i];
             }
+        } else if constexpr (NP == 2) {
+            const float2 u = *reinterpret_cast<const float2 *>(p);
+            x[0] = u.x;
+            x[1] = u.y;
         } else {
 #pragma unroll
             for (int i = 0; i < NP / 4; ++i) {
@@ -128,6 +142,12 @@ template <int NP, int RS> struct RowIn<float, NP, RS> {
                 x[4 * i + 2] = u.z;
                 x[4 * i + 3] = u.w;
             }
+        }
+    }
+    __device__ __forceinline__ void load_each(const float *p) {
+#pragma unroll
+        for (int i = 0; i < NP; ++i) {
+            x[i] = p[RS * i];
         }
     }
     __device__ __forceinline__ float get(int i) const { return x[i]; }
@@ -160,6 +180,8 @@ __device__ __forceinline__ void store_row(T *p, const float (&x)[NP], int kc) {
                         make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
                 }
             }
+        } else if constexpr (NP == 2) {
+            *reinterpret_cast<float2 *>(p) = make_float2(x[0], x[1]);
         } else {
             static_assert(NP % 4 == 0, "whole float4 vectors");
 #pragma unroll
@@ -180,22 +202,16 @@ __device__ __forceinline__ void store_row(T *p, const float (&x)[NP], int kc) {
     }
 }
 
-template <int D, int L, int NP, bool CONTIG, int TPS, typename TQK, typename TV, int GATE>
+template <int D, int L, int NP, typename TQK, typename TV, int GATE>
 __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentArgs a) {
     constexpr int E = D / L;           // K elements per lane
     constexpr int EV = E / 4;          // 16-byte vectors per lane and row
     constexpr int RPW = 64 / L;        // row groups per wave
     constexpr int RPP = 4 * RPW;       // row groups per workgroup
     constexpr int RB = RPP * NP;       // rows per workgroup
-    // A lane's NP rows: consecutive (CONTIG; v and o then move as one vector
-    // per row group) or RPP apart (each wave-wide state load then covers
-    // RPW adjacent rows, one contiguous span).
-    constexpr int RS = CONTIG ? 1 : RPP;
-    // TPS: the tokens per sequence a shape is tuned for -- 1 (decode), 2, or
-    // 3 and more. With several, the token loop's instruction count matters
-    // and the exponentials are one v_exp_f32 each; decode, bound by the
-    // state traffic, keeps the correctly rounded expf.
-    auto dexp = [](float x) { return TPS > 1 ? fexp(x) : expf(x); };
+    // A lane's NP rows are RPP apart: each wave-wide state load covers RPW
+    // adjacent rows, one contiguous span.
+    constexpr int RS = RPP;
     constexpr int VT = D / RB;         // workgroups per (sequence, head)
     static_assert(E % 4 == 0 && D % RB == 0, "whole vectors and whole row tiles");
 
@@ -217,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
     const int wave = threadIdx.x >> 6;
     const int kc = lane % L;
     const int rgw = wave * RPW + lane / L;  // row group in the workgroup
-    const int row0 = vt * RB + (CONTIG ? rgw * NP : rgw);  // rows row0 + RS*p, p < NP
+    const int row0 = vt * RB + rgw;  // rows row0 + RS*p, p < NP
     const int T = a.num_tokens;
 
     int bos = a.cu_seqlens[n];
@@ -357,9 +373,8 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
     };
     // Every row group of a workgroup needs the same per-channel decays, beta
     // and norms of a token. With one vector per lane and row (EV == 1: the
-    // row groups' L lanes cover the D channels four apiece) and one or two
-    // tokens per sequence, the workgroup computes them once and shares them
-    // through LDS: the row groups of the waves before kNormWave each take one
+    // row groups' L lanes cover the D channels four apiece) the workgroup
+    // computes them once and shares them through LDS: the row groups of the waves before kNormWave each take one
     // component of their lanes' vectors (rows groups 0-3: channels 4 kc + r),
     // wave kNormWave forms the q norm (its even row groups) and the k norm
     // (odd ones) with the same group sums every row group would use, and the
@@ -370,7 +385,7 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
     // channel) in the workgroup instead of once per row group (8x fewer).
     // Tokens alternate between two LDS sets, so one barrier per token
     // separates the writes of token t + 2 from the reads of token t.
-    constexpr bool kShare = GATE != KDA_GATE_DECAY && TPS <= 2 && EV == 1;
+    constexpr bool kShare = GATE != KDA_GATE_DECAY && EV == 1;
     constexpr int kNormWave = 4 / RPW;
     static_assert(!kShare || (4 * L == D && kNormWave + 1 < 4), "roles of the shared prologue");
     __shared__ float4 sh_dec[kShare ? 2 : 1][kShare ? L : 1];
@@ -388,9 +403,9 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
                 float d;
                 if constexpr (GATE == KDA_GATE_RAW) {
                     const float db = r == 0 ? dtb[0].x : r == 1 ? dtb[0].y : r == 2 ? dtb[0].z : dtb[0].w;
-                    d = dexp(a.lower_bound / (1.0f + dexp(-(expA * (x + db)))));
+                    d = expf(a.lower_bound / (1.0f + expf(-(expA * (x + db)))));
                 } else {
-                    d = dexp(x);
+                    d = expf(x);
                 }
                 reinterpret_cast<float *>(&sh_dec[par][kc])[r] = d;
             } else if (wave == kNormWave) {
@@ -407,7 +422,7 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
             } else if (wave == kNormWave + 1) {
                 if (kc == 0 && (rgw & (RPW - 1)) == 0) {
                     if constexpr (GATE == KDA_GATE_RAW) {
-                        sh_tok[par][2] = 1.0f / (1.0f + dexp(-in.b));
+                        sh_tok[par][2] = 1.0f / (1.0f + expf(-in.b));
                     } else {
                         sh_tok[par][2] = in.b;
                     }
@@ -437,18 +452,18 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
             if constexpr (GATE == KDA_GATE_RAW) {
                 // g = lower_bound / (1 + exp(-(exp(A_log) * (a + dt_bias)))), decay = exp(g)
                 const float lb = a.lower_bound;
-                w.dec[j].x = dexp(lb / (1.0f + dexp(-(expA * (gv.x + dtb[j].x)))));
-                w.dec[j].y = dexp(lb / (1.0f + dexp(-(expA * (gv.y + dtb[j].y)))));
-                w.dec[j].z = dexp(lb / (1.0f + dexp(-(expA * (gv.z + dtb[j].z)))));
-                w.dec[j].w = dexp(lb / (1.0f + dexp(-(expA * (gv.w + dtb[j].w)))));
+                w.dec[j].x = expf(lb / (1.0f + expf(-(expA * (gv.x + dtb[j].x)))));
+                w.dec[j].y = expf(lb / (1.0f + expf(-(expA * (gv.y + dtb[j].y)))));
+                w.dec[j].z = expf(lb / (1.0f + expf(-(expA * (gv.z + dtb[j].z)))));
+                w.dec[j].w = expf(lb / (1.0f + expf(-(expA * (gv.w + dtb[j].w)))));
             } else if constexpr (GATE == KDA_GATE_LOG) {
-                w.dec[j] = make_float4(dexp(gv.x), dexp(gv.y), dexp(gv.z), dexp(gv.w));
+                w.dec[j] = make_float4(expf(gv.x), expf(gv.y), expf(gv.z), expf(gv.w));
             } else {
                 w.dec[j] = gv;
             }
         }
         if constexpr (GATE == KDA_GATE_RAW) {
-            w.beta = 1.0f / (1.0f + dexp(-in.b));
+            w.beta = 1.0f / (1.0f + expf(-in.b));
         } else {
             w.beta = in.b;
         }
@@ -537,39 +552,20 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
         // every lane of the row group holds the sums
         store_row<TV, NP, RS>(op + (static_cast<int64_t>(t) * H + head) * D + row0, o, kc);
     };
-    if constexpr (TPS > 2) {
-        // One buffer: the next token's loads are issued into it right after
-        // the current token is widened, unconditionally (the last token
-        // reloads itself), so the buffer is always reloaded, never kept --
-        // keeping it would cost register copies and a wait for every
-        // outstanding store on the way back to the loop's top.
-        if (bos < eos) {
-            TokenIn in;
-            fetch(bos, in);
-            for (int t = bos; t < eos; ++t) {
-                Token w;
-                widen(in, w, t);
-                fetch(t + 1 < eos ? t + 1 : t, in);
-                step(w, t);
-            }
+    // Two buffers, the second loaded only when a next token exists (an
+    // unconditional reload would double the token loads of a decode step).
+    TokenIn cur, nxt;
+    if (bos < eos) {
+        fetch(bos, cur);
+    }
+    for (int t = bos; t < eos; ++t) {
+        if (t + 1 < eos) {
+            fetch(t + 1, nxt);
         }
-    } else {
-        // One or two tokens per sequence: a second buffer, loaded only when
-        // a next token exists (an unconditional reload would be a third of
-        // the token loads at two tokens, all of them at one).
-        TokenIn cur, nxt;
-        if (bos < eos) {
-            fetch(bos, cur);
-        }
-        for (int t = bos; t < eos; ++t) {
-            if (t + 1 < eos) {
-                fetch(t + 1, nxt);
-            }
-            Token w;
-            widen(cur, w, t);
-            step(w, t);
-            cur = nxt;
-        }
+        Token w;
+        widen(cur, w, t);
+        step(w, t);
+        cur = nxt;
     }
 
     // Tokens no sequence covers are zero (the reference allocates
@@ -602,27 +598,454 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
     }
 }
 
+// ---------------------------------------------------------------------------
+// Several tokens per sequence (verify, short prefill): tokens in blocks.
+//
+// What bounds the token loop is VALU issue: four multiply-adds per state
+// element and token (65 us for 1169 tokens on 32 heads at the unpacked fp32
+// rate), and before them the token's gates and norms, which every row group
+// of the workgroup needs alike (about 350 of 550 instructions per token and
+// wave when each forms them for itself). So they are formed once per
+// workgroup: of a block of 16 tokens, 16-lane row group i loads token i (q,
+// k, gate, beta and the tile's v rows), forms the decays, the normalized k
+// and the scaled q, and leaves them in LDS; after one barrier every row group
+// steps through the block's tokens reading ready values. The next block's
+// inputs are loaded behind the barrier and wait in registers while the tokens
+// run, and a token's outputs replace its v values in LDS, from where the
+// block's rows leave as vectors. 16 requests of 20-120 tokens, H=32, raw
+// gates: 253 -> 115 us; 2 x 63 tokens, H=4, D=64, fp32: 42 -> 17 us; 256 x 8
+// tokens, H=32: 307 -> 210 us.
+//
+// SW: the waves that share a block. 4: the workgroup, 16 tokens a block. 1:
+// each wave for its own rows, four tokens a block and no barrier, for few
+// tokens on many pairs, where the state's traffic is the bound and a barrier
+// only makes the waves' loads wait for each other.
+// Row groups of 16 lanes, a lane owning D / 16 K elements of NP consecutive
+// rows; a workgroup covers 16 NP rows.
+// ---------------------------------------------------------------------------
+
+template <int D, int NP, int SW, typename TQK, typename TV, int GATE>
+__global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const KdaRecurrentArgs a) {
+    constexpr int L = 16;
+    constexpr int EV = D / L / 4;  // 16-byte vectors per lane and row
+    constexpr int RB = 16 * NP;    // rows per workgroup
+    constexpr int VT = D / RB;     // workgroups per (sequence, head)
+    constexpr int BTOK = 4 * SW;   // tokens per block: a row group of the sharing waves each
+    constexpr int SR = BTOK * NP;  // rows of the sharing waves
+    constexpr int VP = SR / L;     // v values a lane stages
+    static_assert(D % RB == 0 && (SW == 1 || SW == 4) && VP >= 1, "whole row tiles");
+    // D = 64 keeps the correctly rounded expf of its one-token form.
+    auto dexp = [](float x) { return D == 128 ? fexp(x) : expf(x); };
+
+    // one block's prepared tokens: [token][channel], and [token][row of the
+    // tile]: v before the token's step, its output after
+    __shared__ float4 all_k[4 / SW][BTOK][D / 4];
+    __shared__ float4 all_q[4 / SW][BTOK][D / 4];
+    __shared__ float4 all_dec[4 / SW][BTOK][D / 4];
+    __shared__ float all_beta[4 / SW][BTOK];
+    __shared__ alignas(16) float all_vo[4 / SW][BTOK][SR];
+
+    const int H = a.num_heads;
+    const int HC = a.head_count;
+    // XCD-aware order, as in recurrent_kernel
+    const int b = blockIdx.x;
+    const int rest = b >> 3;
+    const int vt = VT == 1 ? 0 : rest % VT;
+    const int pair = VT == 1 ? b : (rest / VT) * 8 + (b & 7);
+    const int n = pair / HC;
+    const int head = a.head_begin + (pair - n * HC);
+    if (n >= a.num_seqs) {
+        return;
+    }
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kc = lane % L;
+    // row group among the sharing waves; in the prologue, the block's token
+    const int rg = SW == 1 ? lane / L : static_cast<int>(threadIdx.x) / L;
+    const int share = SW == 1 ? wave : 0;
+    const int base0 = vt * RB + share * SR;  // the sharing waves' first row
+    const int row0 = base0 + rg * NP;
+    auto &sh_k = all_k[share];
+    auto &sh_q = all_q[share];
+    auto &sh_dec = all_dec[share];
+    auto &sh_beta = all_beta[share];
+    auto &sh_vo = all_vo[share];
+    auto sync = [&]() {
+        if constexpr (SW == 4) {
+            lds_barrier();
+        } else {
+            // one wave's LDS accesses happen in order
+            asm volatile("" ::: "memory");
+        }
+    };
+    const int T = a.num_tokens;
+
+    int bos = a.cu_seqlens[n];
+    int eos = a.cu_seqlens[n + 1];
+    bos = bos < 0 ? 0 : (bos > T ? T : bos);
+    eos = eos < bos ? bos : (eos > T ? T : eos);
+    int slot = a.state_indices[n];
+    if (slot < 0 || static_cast<int64_t>(slot) >= a.num_slots) {
+        slot = 0;
+    }
+
+    auto koff = [&](int j) { return 4 * kc + 4 * L * j; };
+    const TQK *qp = static_cast<const TQK *>(a.q);
+    const TQK *kp = static_cast<const TQK *>(a.k);
+    const TV *vp = static_cast<const TV *>(a.v);
+    TV *op = static_cast<TV *>(a.out);
+    using TG = typename std::conditional<GATE == KDA_GATE_RAW, uint16_t, float>::type;
+    const TG *gp = static_cast<const TG *>(a.gate);
+
+    // Inputs of this row group's token of the block at t0 (the last token's
+    // where the block has fewer: loaded, prepared and never used). A wave
+    // none of whose four tokens exists loads nothing.
+    Raw4<TQK> rq[EV], rk[EV];
+    Raw4<TG> rgate[EV];
+    RowIn<TV, VP, VP == 1 ? 16 : 1> rv;
+    // v and out may sit anywhere: whole vectors where both are aligned for
+    // them, element by element otherwise
+    constexpr uintptr_t kVecBytes = VP * sizeof(TV) > 16 ? 16 : VP * sizeof(TV);
+    const bool vec = ((reinterpret_cast<uintptr_t>(vp) | reinterpret_cast<uintptr_t>(op)) & (kVecBytes - 1)) == 0;
+    float rb = 0.f;
+    auto fetch = [&](int t0) {
+        if (t0 + (SW == 1 ? 0 : 4 * wave) < eos) {
+            const int t = t0 + rg < eos ? t0 + rg : eos - 1;
+            const int64_t bi = static_cast<int64_t>(t) * H + head;
+            const int64_t base = bi * D;
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                rq[j].load(qp + base + koff(j));
+                rk[j].load(kp + base + koff(j));
+                rgate[j].load(gp + base + koff(j));
+            }
+            if (vec) {
+                rv.load(vp + base + base0 + kc * VP);
+            } else {
+                rv.load_each(vp + base + base0 + kc * VP);
+            }
+            if constexpr (GATE == KDA_GATE_RAW) {
+                rb = bf16_to_f32(static_cast<const uint16_t *>(a.beta)[bi]);
+            } else {
+                rb = static_cast<const float *>(a.beta)[bi];
+            }
+        }
+    };
+    // Raw gates: the inputs' loads go ahead of the state's, whose wait would
+    // otherwise cover them, since the prologue is long (512 x 2 tokens, H=32,
+    // one wave sharing: 356 us, against 377 behind them). Prepared gates have
+    // a short prologue, and with one wave sharing the state goes first
+    // (1024 x 4 tokens, H=16: 373 us, against 389).
+    constexpr bool kInputsFirst = SW == 4 || GATE == KDA_GATE_RAW;
+    if (kInputsFirst && bos < eos) {
+        fetch(bos);
+    }
+
+    const int64_t head_off = static_cast<int64_t>(head) * a.state_stride_head;
+    const bool vpool = GATE == KDA_GATE_DECAY && a.state_v_contiguous != 0;
+    float4 S[NP][EV];
+    if (slot > 0) {
+        const float *src = a.state + slot * a.state_stride_slot + head_off;
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                if (vpool) {
+                    const float *e = src + static_cast<int64_t>(koff(j)) * D + row0 + p;
+                    S[p][j] = make_float4(e[0], e[D], e[2 * D], e[3 * D]);
+                } else {
+                    S[p][j] = load4_stream(src + static_cast<int64_t>(row0 + p) * D + koff(j));
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                S[p][j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        }
+    }
+
+    if (!kInputsFirst && bos < eos) {
+        fetch(bos);
+    }
+
+    int track_slot = 0;
+    int track_len = -1;
+    if (a.track_indices != nullptr) {
+        track_slot = a.track_indices[n];
+        if (track_slot <= 0 || static_cast<int64_t>(track_slot) >= a.num_slots) {
+            track_slot = 0;
+        } else {
+            track_len = a.track_lens[n];
+        }
+    }
+    auto store_state = [&](float *dst, bool vlayout) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                if (vlayout) {
+                    float *e = dst + static_cast<int64_t>(koff(j)) * D + row0 + p;
+                    e[0] = S[p][j].x;
+                    e[D] = S[p][j].y;
+                    e[2 * D] = S[p][j].z;
+                    e[3 * D] = S[p][j].w;
+                } else {
+                    store4_stream(dst + static_cast<int64_t>(row0 + p) * D + koff(j), S[p][j]);
+                }
+            }
+        }
+    };
+    if (track_slot > 0 && track_len == 0) {
+        store_state(a.state + track_slot * a.state_stride_slot + head_off, vpool);
+    }
+
+    float expA = 0.f;
+    if constexpr (GATE == KDA_GATE_RAW) {
+        expA = expf(a.A_log[head]);
+    }
+    const bool norm = (GATE == KDA_GATE_RAW) || (a.qk_l2norm != 0);
+    const bool save_mid = a.intermediate != nullptr && slot > 0 && n < a.mid_rows;
+
+    // the fetched token, prepared, into LDS
+    auto prepare = [&](int t0) {
+        if (t0 + (SW == 1 ? 0 : 4 * wave) >= eos) {
+            return;
+        }
+        float4 q[EV], k[EV], dec[EV];
+#pragma unroll
+        for (int j = 0; j < EV; ++j) {
+            q[j] = rq[j].get();
+            k[j] = rk[j].get();
+            const float4 gv = rgate[j].get();
+            if constexpr (GATE == KDA_GATE_RAW) {
+                // g = lower_bound / (1 + exp(-(exp(A_log) * (a + dt_bias)))), decay = exp(g)
+                const float lb = a.lower_bound;
+                const float4 dtb = load4(a.dt_bias + static_cast<int64_t>(head) * D + koff(j));
+                dec[j].x = dexp(lb / (1.0f + dexp(-(expA * (gv.x + dtb.x)))));
+                dec[j].y = dexp(lb / (1.0f + dexp(-(expA * (gv.y + dtb.y)))));
+                dec[j].z = dexp(lb / (1.0f + dexp(-(expA * (gv.z + dtb.z)))));
+                dec[j].w = dexp(lb / (1.0f + dexp(-(expA * (gv.w + dtb.w)))));
+            } else if constexpr (GATE == KDA_GATE_LOG) {
+                dec[j] = make_float4(dexp(gv.x), dexp(gv.y), dexp(gv.z), dexp(gv.w));
+            } else {
+                dec[j] = gv;
+            }
+        }
+        float qsc = a.scale;
+        float kr = 1.f;
+        if (norm) {
+            // x / sqrt(sum x^2 + 1e-6), eps inside the sqrt; q then scaled.
+            float qs = 0.f, ks = 0.f;
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                qs += dot4(q[j], q[j]);
+                ks += dot4(k[j], k[j]);
+            }
+            qs = group_sum<L>(qs);
+            ks = group_sum<L>(ks);
+            kr = 1.0f / sqrtf(ks + 1e-6f);
+            qsc = (1.0f / sqrtf(qs + 1e-6f)) * a.scale;
+        }
+#pragma unroll
+        for (int j = 0; j < EV; ++j) {
+            sh_k[rg][kc + L * j] = make_float4(k[j].x * kr, k[j].y * kr, k[j].z * kr, k[j].w * kr);
+            sh_q[rg][kc + L * j] = make_float4(q[j].x * qsc, q[j].y * qsc, q[j].z * qsc, q[j].w * qsc);
+            sh_dec[rg][kc + L * j] = dec[j];
+        }
+#pragma unroll
+        for (int p = 0; p < VP; ++p) {
+            sh_vo[rg][kc * VP + p] = rv.get(p);
+        }
+        if (kc == 0) {
+            if constexpr (GATE == KDA_GATE_RAW) {
+                sh_beta[rg] = 1.0f / (1.0f + dexp(-rb));
+            } else {
+                sh_beta[rg] = rb;
+            }
+        }
+    };
+    struct Token {
+        float4 k[EV], dec[EV], q[EV];
+        float beta;
+        float v[NP];
+    };
+    auto read = [&](Token &w, int i) {
+#pragma unroll
+        for (int j = 0; j < EV; ++j) {
+            w.dec[j] = sh_dec[i][kc + L * j];
+            w.k[j] = sh_k[i][kc + L * j];
+            w.q[j] = sh_q[i][kc + L * j];
+        }
+        w.beta = sh_beta[i];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            w.v[p] = sh_vo[i][rg * NP + p];
+        }
+    };
+    // sum over the lane's elements of s * x, one multiply-add chain
+    auto dot_lane = [](const float4 (&sv)[EV], const float4 (&xv)[EV]) {
+        float acc = dot4(sv[0], xv[0]);
+#pragma unroll
+        for (int j = 1; j < EV; ++j) {
+            acc = fmaf(sv[j].x, xv[j].x, acc);
+            acc = fmaf(sv[j].y, xv[j].y, acc);
+            acc = fmaf(sv[j].z, xv[j].z, acc);
+            acc = fmaf(sv[j].w, xv[j].w, acc);
+        }
+        return acc;
+    };
+    auto step = [&](const Token &w, int i, int step_i) {
+        float pred[NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                S[p][j].x *= w.dec[j].x;
+                S[p][j].y *= w.dec[j].y;
+                S[p][j].z *= w.dec[j].z;
+                S[p][j].w *= w.dec[j].w;
+            }
+            pred[p] = dot_lane(S[p], w.k);
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            pred[p] = group_sum<L>(pred[p]);
+        }
+        float o[NP];
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            const float d = (w.v[p] - pred[p]) * w.beta;
+#pragma unroll
+            for (int j = 0; j < EV; ++j) {
+                S[p][j].x += w.k[j].x * d;
+                S[p][j].y += w.k[j].y * d;
+                S[p][j].z += w.k[j].z * d;
+                S[p][j].w += w.k[j].w * d;
+            }
+            o[p] = dot_lane(S[p], w.q);
+        }
+        if (save_mid && step_i < a.mid_steps) {
+            store_state(a.intermediate + n * a.mid_stride_req + step_i * a.mid_stride_step +
+                            static_cast<int64_t>(head) * a.mid_stride_head,
+                        false);
+        }
+        if (track_slot > 0 && step_i + 1 == track_len) {
+            store_state(a.state + track_slot * a.state_stride_slot + head_off, vpool);
+        }
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            o[p] = group_sum<L>(o[p]);
+        }
+        if (kc == 0) {  // every lane of the row group holds the sums
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+                sh_vo[i][rg * NP + p] = o[p];
+            }
+        }
+    };
+    // the final state, ahead of the last block's outputs
+    auto finish = [&]() {
+        if (a.intermediate == nullptr && slot > 0) {
+            store_state(a.state + slot * a.state_stride_slot + head_off, vpool);
+        }
+    };
+    if (bos >= eos) {
+        finish();
+    }
+    for (int t0 = bos; t0 < eos; t0 += BTOK) {
+        prepare(t0);
+        sync();
+        if (t0 + BTOK < eos) {
+            fetch(t0 + BTOK);
+        }
+        const int len = eos - t0 < BTOK ? eos - t0 : BTOK;
+        if constexpr (NP == 1) {
+            Token cur;
+            read(cur, 0);
+            for (int i = 0; i < len; ++i) {
+                Token nxt;
+                read(nxt, i + 1 < len ? i + 1 : i);
+                step(cur, i, t0 - bos + i);
+                cur = nxt;
+            }
+        } else {
+            for (int i = 0; i < len; ++i) {
+                Token cur;
+                read(cur, i);
+                step(cur, i, t0 - bos + i);
+            }
+        }
+        if (t0 + BTOK >= eos) {
+            finish();
+        }
+        sync();
+        // the block's outputs, token rg by row group rg, which also rewrites
+        // exactly these entries for the next block
+        if (rg < len) {
+            float o[VP];
+#pragma unroll
+            for (int p = 0; p < VP; ++p) {
+                o[p] = sh_vo[rg][kc * VP + p];
+            }
+            TV *dst = op + (static_cast<int64_t>(t0 + rg) * H + head) * D + base0 + kc * VP;
+            if (VP > 1 && vec) {
+                store_row<TV, VP, VP == 1 ? 16 : 1>(dst, o, kc);
+            } else {
+#pragma unroll
+                for (int p = 0; p < VP; ++p) {
+                    store1(dst + p, o[p]);
+                }
+            }
+        }
+    }
+
+    // rows no request covers, as in recurrent_kernel
+    auto zero_rows = [&](int ta, int tb) {
+        for (int t = ta + rg; t < tb; t += BTOK) {
+#pragma unroll
+            for (int p = 0; p < VP; ++p) {
+                store1(op + (static_cast<int64_t>(t) * H + head) * D + base0 + kc * VP + p, 0.f);
+            }
+        }
+    };
+    if constexpr (GATE != KDA_GATE_DECAY) {
+        if (n == 0) {
+            zero_rows(0, bos);
+        }
+        if (n == a.num_seqs - 1) {
+            zero_rows(eos, T);
+        }
+    }
+
+}
+
 using KernelFn = void (*)(const KdaRecurrentArgs);
 
 // Tile shapes: (lanes per row L, rows per lane NP).
-enum Shape { kDecode16, kDecode8, kVerify16, kMulti32, kMulti64, kMulti128, kD64Small, kD64Large };
+enum Shape { kDecode16, kDecode8, kBlock16, kBlock64, kBlock128, kWave128, kD64Small, kD64Large };
 
 template <int D, typename TQK, typename TV, int GATE>
 KernelFn pick_shape(Shape shape) {
     if constexpr (D == 128) {
         switch (shape) {
-            case kDecode16: return recurrent_kernel<D, 32, 2, false, 1, TQK, TV, GATE>;
-            case kDecode8: return recurrent_kernel<D, 32, 1, false, 1, TQK, TV, GATE>;
-            case kVerify16: return recurrent_kernel<D, 16, 1, false, 3, TQK, TV, GATE>;
-            case kMulti32: return recurrent_kernel<D, 32, 4, false, 2, TQK, TV, GATE>;
-            case kMulti64: return recurrent_kernel<D, 16, 4, true, 3, TQK, TV, GATE>;
-            case kMulti128: return recurrent_kernel<D, 16, 8, true, 3, TQK, TV, GATE>;
+            case kDecode16: return recurrent_kernel<D, 32, 2, TQK, TV, GATE>;
+            case kDecode8: return recurrent_kernel<D, 32, 1, TQK, TV, GATE>;
+            case kBlock16: return recurrent_block_kernel<D, 1, 4, TQK, TV, GATE>;
+            case kBlock64: return recurrent_block_kernel<D, 4, 4, TQK, TV, GATE>;
+            case kBlock128: return recurrent_block_kernel<D, 8, 4, TQK, TV, GATE>;
+            case kWave128: return recurrent_block_kernel<D, 8, 1, TQK, TV, GATE>;
             default: return nullptr;
         }
     } else {
         switch (shape) {
-            case kD64Large: return recurrent_kernel<D, 16, 4, false, 1, TQK, TV, GATE>;
-            case kD64Small: return recurrent_kernel<D, 16, 1, false, 1, TQK, TV, GATE>;
+            case kD64Large: return recurrent_kernel<D, 16, 4, TQK, TV, GATE>;
+            case kD64Small: return recurrent_kernel<D, 16, 1, TQK, TV, GATE>;
+            case kBlock16: return recurrent_block_kernel<D, 1, 4, TQK, TV, GATE>;
+            case kBlock64: return recurrent_block_kernel<D, 4, 4, TQK, TV, GATE>;
             default: return nullptr;
         }
     }
@@ -719,62 +1142,57 @@ extern "C" int kda_recurrent_launch(const KdaRecurrentArgs *args, void *stream) 
     if (kargs.head_count == 0 || kargs.head_begin + kargs.head_count > kargs.num_heads) {
         kargs.head_count = kargs.num_heads - kargs.head_begin;
     }
-    // Tile shape at D=128, by tokens per sequence (measured on MI355X,
-    // interleaved A/B on one box): one token (decode) -> 32-lane rows, 2 rows
-    // per lane: 16-row tiles, eight workgroups per (sequence, head), which
-    // stream the state fastest (B=256, H=32: 173 us, against 182 with
-    // 32-row tiles); two tokens -> 32-lane rows, 4 rows per lane (32-row
-    // tiles: 361 us at 512 x 2 tokens, H=32, against 367 with 16-lane
-    // rows); more (verify, recurrent prefill) -> 16-lane rows, whose
-    // reductions take four DPP steps instead of five plus a swizzle, with 8
-    // consecutive rows per lane (the whole state of a (sequence, head) in one
-    // workgroup) so each token's loads and exponentials serve more rows:
-    // 1024 x 4 tokens, H=16: 382 us, against 406 with 4 rows per lane, 464
-    // with 2 and 432 with 32-lane rows; 256 x 8 tokens, H=32: 265 against
-    // 284 and 351. The 8-row-per-lane shape runs three workgroups per CU, so
-    // below 1024 pairs the 4-row one (two workgroups per pair) fills the GPU
-    // instead. Fewer than 128 pairs: one token per request uses 8-row tiles,
-    // 32 lanes per row; several (speculative verify) use 16-row tiles of
-    // 16-lane rows with the multi-token loop (2 requests x 4 tokens, H=32:
-    // 8.7 us against 12.8 with the decode shape).
+    // Tile shape at D=128, by tokens per sequence and (sequence, head) pairs
+    // (measured on MI355X as graph replays, microseconds; "loop" is a token
+    // loop without shared blocks, which these shapes replaced).
+    // One token (decode): 32-lane rows, 2 rows per lane: 16-row tiles, eight
+    // workgroups per pair, which stream the state fastest (B=256, H=32: 173,
+    // against 182 with 32-row tiles); 8-row tiles below 128 pairs.
+    // Several tokens: blocks. Below 128 pairs 16-row tiles, whose eight
+    // workgroups per pair spread a short step over the CUs (2 x 4 tokens,
+    // H=32, checkpoints: 6.2, against 6.8 with 64-row tiles; loop 9.2). While
+    // all of them are resident at once (four workgroups of two per pair and
+    // CU, three with fp32 inputs' registers) 64-row tiles (16 x 20-120
+    // tokens, H=32: 115, against 147 with 128-row tiles; loop 253). Beyond,
+    // short sequences take 128-row tiles, which prepare a token once per pair
+    // and run in fewer rounds (48 x 4 tokens, H=16: 17.7 against 21.2; loop
+    // 27.2), long ones, bound by VALU issue, keep the 64-row tiles' higher
+    // occupancy (64 x 20-120 tokens, H=32: 399 against 414; loop 728). With
+    // 2048 pairs and more the state's traffic bounds a few tokens: up to four
+    // no barrier is worth its coupling of the waves' loads (one wave sharing,
+    // 512 x 4 tokens, H=32: 353, against 389; loop 383), up to six the 64-row
+    // tiles stream better (256 x 6, H=32, prepared gates: 191 against 196 and
+    // 215 with one wave sharing; loop 201).
+    // D=64: 64-row tiles are one workgroup per pair, 16-row tiles four (2 x
+    // 37-63 tokens, H=4: 17 against 25; 64 x 4, H=16: 14.9 against 9.1).
     const int64_t pairs = static_cast<int64_t>(a.num_seqs) * kargs.head_count;
+    const int64_t seqs = a.num_seqs;
+    const int64_t ntok = a.num_tokens;
     Shape shape;
-    int rows_per_wg;
     if (D == 128) {
-        const int64_t tokens = a.num_tokens;
-        if (pairs < 128) {
-            shape = tokens <= a.num_seqs ? kDecode8 : kVerify16;
-        } else if (tokens <= a.num_seqs) {
-            shape = kDecode16;
-        } else if (tokens <= 2 * static_cast<int64_t>(a.num_seqs)) {
-            shape = kMulti32;
-        } else if (pairs < 1024) {
-            shape = kMulti64;
+        const int64_t resident = a.qk_dtype == KDA_F32 ? 384 : 512;
+        if (ntok <= seqs) {
+            shape = pairs < 128 ? kDecode8 : kDecode16;
+        } else if (pairs < 128) {
+            shape = kBlock16;
+        } else if (pairs <= resident || ntok > 16 * seqs) {
+            shape = kBlock64;
+        } else if (pairs < 2048 || ntok > 6 * seqs) {
+            shape = kBlock128;
         } else {
-            shape = kMulti128;
+            shape = ntok <= 4 * seqs ? kWave128 : kBlock64;
         }
-        // The 16-lane shapes move a lane's consecutive v and o values as one
-        // vector of up to 16 bytes; v or out not aligned for that take the
-        // 32-row shape, which moves them one element at a time.
-        if (shape == kMulti64 || shape == kMulti128) {
-            const size_t vbytes = static_cast<size_t>(shape == kMulti128 ? 8 : 4) *
-                                  (a.v_dtype == KDA_F32 ? 4 : 2);
-            const uintptr_t mis = (reinterpret_cast<uintptr_t>(a.v) |
-                                   reinterpret_cast<uintptr_t>(a.out)) &
-                                  ((vbytes > 16 ? 16 : vbytes) - 1);
-            if (mis != 0) {
-                shape = kMulti32;
-            }
-        }
-        rows_per_wg = shape == kDecode8    ? 8
-                      : shape == kVerify16 ? 16
-                      : shape == kDecode16 ? 16
-                      : shape == kMulti32  ? 32
-                      : shape == kMulti64  ? 64
-                                           : 128;
-    } else {
+    } else if (ntok <= seqs) {
         shape = pairs >= 2048 ? kD64Large : kD64Small;
-        rows_per_wg = shape == kD64Large ? 64 : 16;
+    } else {
+        shape = pairs >= 256 ? kBlock64 : kBlock16;
+    }
+    int rows_per_wg = 128;
+    switch (shape) {
+        case kDecode8: rows_per_wg = 8; break;
+        case kDecode16: case kBlock16: case kD64Small: rows_per_wg = 16; break;
+        case kBlock64: case kD64Large: rows_per_wg = 64; break;
+        case kBlock128: case kWave128: break;
     }
     KernelFn fn = (D == 128) ? pick_kernel<128>(a.gate_mode, a.qk_dtype, a.v_dtype, shape)
                              : pick_kernel<64>(a.gate_mode, a.qk_dtype, a.v_dtype, shape);
