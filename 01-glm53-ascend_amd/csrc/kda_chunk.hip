@@ -101,12 +101,11 @@ constexpr int kOffSc = kOffGl + DK * 4;           // fp32 scale block [128], ind
 constexpr int kRecBytes = kOffSc + 512;           // 56320
 // Scale block: 2^-shift of each fp16 fragment group, and the bound the scan
 // derives y's scale from (|y| <= max|v| + kel1 max|S|).
-constexpr int kScKe = 0;     // [16] e^G k fragment (mt, s): mt * 4 + s (equal within s = 0, 1 and s = 2, 3)
-constexpr int kScQg = 16;    // [16] q e^G fragment (mt, s) (equal within s = 0, 1 and s = 2, 3)
-constexpr int kScKd = 32;    // [8]  (T^T kd)^T row tile mk (both token slices)
-constexpr int kScAq = 40;    // [4]  Aqk T row tile mt (both token slices)
-constexpr int kScKel1 = 48;  // [8]  4 h + mt: max over the rows t of tile mt of the sum of
-                             //      |(e^G k)[t][k]| over channel half h (k in [64h, 64h + 64))
+constexpr int kScKe = 0;     // [1] e^G k, all fragments
+constexpr int kScQg = 1;     // [1] q e^G, all fragments
+constexpr int kScKel1 = 2;   // [1] a bound of max_t sum_k |(e^G k)[t][k]|
+constexpr int kScKd = 32;    // [8] (T^T kd)^T row tile mk (both token slices)
+constexpr int kScAq = 40;    // [4] Aqk T row tile mt (both token slices)
 // Largest of four nonnegative values (magnitudes), compared as their bit
 // patterns: no quieting of the operands as fmaxf needs for values it did not
 // produce itself.
@@ -115,14 +114,6 @@ __device__ __forceinline__ float max4_mag(float a, float b, float c, float d) {
                                max(__float_as_uint(c), __float_as_uint(d))));
 }
 __device__ __forceinline__ float max4_mag(float4 v) { return max4_mag(v.x, v.y, v.z, v.w); }
-
-// max over a chunk's rows t of sum_k |(e^G k)[t][k]|, bounded from above by
-// the two channel halves' maxima of each row tile
-__device__ __forceinline__ float kel1_bound(const float *sc) {
-    const float4 h0 = *reinterpret_cast<const float4 *>(sc + kScKel1);
-    const float4 h1 = *reinterpret_cast<const float4 *>(sc + kScKel1 + 4);
-    return max4_mag(h0.x + h1.x, h0.y + h1.y, h0.z + h1.z, h0.w + h1.w);
-}
 
 // Track record of one (sequence, head): operands of the state after r < len
 // tokens of the chunk holding the tracked position.
@@ -200,6 +191,18 @@ __device__ __forceinline__ uint32_t pack2(uint16_t lo, uint16_t hi) {
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 __device__ __forceinline__ u32x4 as_u32x4(bf16x8 v) { return __builtin_bit_cast(u32x4, v); }
 
+// x - h for h one half of a bf16 pair (exact when h is x rounded): one
+// v_dot2_f32_bf16 of the pair with (-1, 0) or (0, -1), where widening the half
+// and subtracting take two instructions.
+template <int HALF>
+__device__ __forceinline__ float bf16_residual(float x, uint32_t hp) {
+    typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    uint32_t sel = HALF == 0 ? 0x0000bf80u : 0xbf800000u;
+    asm("" : "+s"(sel));  // from a register: as the inline constant -1.0 the first one was read as the second
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_t, hp), __builtin_bit_cast(bf16x2_t, sel), x,
+                                           false);
+}
+
 // x[8] -> bf16 hi (+ lo) fragments; lo = bf16(x - hi), so x = hi + lo to
 // about 2^-17 relative.
 __device__ __forceinline__ bf16x8 to_bf16x8(const float x[8]) {
@@ -215,10 +218,8 @@ __device__ __forceinline__ void split_bf16x8(const float x[8], bf16x8 &hi, bf16x
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         const uint32_t hp = pack_bf16x2(x[2 * p], x[2 * p + 1]);
-        const float h0 = __uint_as_float(hp << 16);
-        const float h1 = __uint_as_float(hp & 0xffff0000u);
         h[p] = hp;
-        l[p] = pack_bf16x2(x[2 * p] - h0, x[2 * p + 1] - h1);
+        l[p] = pack_bf16x2(bf16_residual<0>(x[2 * p], hp), bf16_residual<1>(x[2 * p + 1], hp));
     }
     hi = as_bf16x8(h);
     lo = as_bf16x8(l);
@@ -298,32 +299,27 @@ __device__ __forceinline__ float wave_max_mag(float x) {
     return __uint_as_float(max(a, b));
 }
 
-// One wave stores NF consecutive fp16 fragments with one shared scale, and
-// writes the inverse scale to sc[0 .. nsc).
+// Per 16-bit half, the larger of m and the magnitude of a bf16 value (as bits).
+__device__ __forceinline__ uint32_t max_mag_bf16x2(uint32_t m, uint32_t x) {
+    typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, m),
+                                                                  __builtin_bit_cast(u16x2_t, x & 0x7fff7fffu)));
+}
+
+// One wave stores NF consecutive fp16 fragments of x * 2^sh.
 template <int NF>
-__device__ __forceinline__ void store_frags_f16(char *base, int off, int idx, float *sc, int lane,
-                                                const float (&x)[NF][8], int nsc = 1) {
-    float m = 0.f;
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            m = fmaxf(m, fabsf(x[f][e]));
-        }
-    }
-    const int sh = f16_shift(wave_max_mag(m));
+__device__ __forceinline__ void store_frags_f16(char *base, int off, int idx, int sh, int lane,
+                                                const float (&x)[NF][8]) {
 #pragma unroll
     for (int f = 0; f < NF; ++f) {
         reinterpret_cast<u32x4 *>(base + off)[(idx + f) * 64 + lane] = as_u32x4(to_f16x8(x[f], sh));
     }
-    if (lane < nsc) {
-        sc[lane] = ldexpf(1.f, -sh);
-    }
 }
 
-// store_frags_f16 for values given as x * 2^ex[t], with t = 2f + (e >= 4) the
-// 16-row tile of element e of fragment f: the exponents join the fragment's
-// own shift (one ldexp per value; power-of-two factors change no bits).
+// One wave stores NF consecutive fp16 fragments with one shared scale, written
+// inverted to sc[0], of values given as x * 2^ex[t], with t = 2f + (e >= 4) the
+// 16-row tile of element e of fragment f: the exponents join the shared
+// shift (one ldexp per value; power-of-two factors change no bits).
 template <int NF>
 __device__ __forceinline__ void store_frags_f16_exp(char *base, int off, int idx, float *sc, int lane,
                                                     const float (&x)[NF][8], const int (&ex)[2 * NF]) {
@@ -554,10 +550,9 @@ constexpr int kPadX = 68;   // fp32 row stride of [64][64] tiles (16-B rows)
 
 __device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Akk / Aqk exponent anchor: row 7 of each 16-row block, and the largest
-// exponent (log2 units) a factor may take before it is clamped. A chunk in
-// which some block's factors would span more than kExactExp2 (the margin
-// covers the rounding of the cumsum) takes the exact form instead.
+// Akk / Aqk exponent anchor: row 7 of each 16-row block. A chunk in which some
+// block's factors would span more than kExactExp2 (the margin to kMaxExp2, where
+// fp32 ends, covers the rounding of the cumsum) takes the exact form instead.
 constexpr int kAnchorRow = 7;
 constexpr float kMaxExp2 = 126.f;
 constexpr float kExactExp2 = 125.f;
@@ -595,7 +590,13 @@ struct PrepShared {
     } u;
     float beta[BT];
     float gsum[4][DK];  // each wave's two row groups' decay sums (the cumsum's carries)
-    alignas(16) int far[4];  // per wave: some anchor factor of its rows spans > kExactExp2
+    alignas(16) int far[4];     // per wave: some anchor factor of its rows spans > kExactExp2
+    // per wave: largest magnitude of its k and q rows as given (bf16 bits; not
+    // used when they are normalized), largest positive log2 decay of a token
+    // (0 for decays, which are <= 0)
+    alignas(16) uint32_t kmax[4];
+    alignas(16) uint32_t qmax[4];
+    alignas(16) float grow[4];
 };
 static_assert(sizeof(PrepShared) <= 80 * 1024, "two prepare workgroups per CU");
 
@@ -788,6 +789,29 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             *reinterpret_cast<float4 *>(&sm.u.early.K[t][4 * kc]) =
                 make_float4(k4.x * rn, k4.y * rn, k4.z * rn, k4.w * rn);
         }
+        // The extremes the record's fp16 scales are bounded by: max |k|, and how
+        // far a token's decay goes above 1 (never, when g <= 0)
+        if (!norm) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                m = max_mag_bf16x2(max_mag_bf16x2(m, kraw[i].x), kraw[i].y);
+            }
+            sm.kmax[wave] = __float_as_uint(wave_max_mag(__uint_as_float(max(m & 0xffffu, m >> 16))));
+        }
+        {
+            int m = 0;  // positive floats order as their bits, negative ones are below 0
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                m = max(max(max(m, __float_as_int(g4[i].x)), __float_as_int(g4[i].y)),
+                        max(__float_as_int(g4[i].z), __float_as_int(g4[i].w)));
+            }
+            float up = 0.f;
+            if (__builtin_expect(__ballot(m > 0) != 0ull, 0)) {
+                up = wave_max_mag(__int_as_float(m)) * kLog2e;
+            }
+            sm.grow[wave] = up;
+        }
         // S2, the in-chunk cumsum of the log2 decay: this lane's eight rows in
         // registers, then the row groups before it: its half-wave partner
         // (rg - 1, for odd rg) by a lane exchange, earlier waves' pairs
@@ -868,8 +892,52 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 sm.u.early.qss[sh][16 * (ii == 0 ? IA : 3 - IA) + r] = ss;
             }
         }
+    } else {
+        uint32_t m = 0;
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii) {
+#pragma unroll
+            for (int q2 = 0; q2 < 2; ++q2) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    m = max_mag_bf16x2(max_mag_bf16x2(m, qraw[ii][q2][e].x), qraw[ii][q2][e].y);
+                }
+            }
+        }
+        sm.qmax[wave] = __float_as_uint(wave_max_mag(__uint_as_float(max(m & 0xffffu, m >> 16))));
     }
     lds_barrier();
+
+    // Power-of-two scales of the record's fp16 operands from bounds rather than
+    // from their own largest values, whose search cost K1 a reduction over the
+    // wave per fragment group (six of them, and 60 maxima per lane): |e^G k| and
+    // |kd| <= max|k|, |q e^G| <= max|q|, |Aqk| <= 128 max|k| max|q| (all times
+    // 2^up where a decay goes above 1); normalized rows have norm 1. fp16
+    // keeps its 11 bits down to 2^-28 of the bound, so a bound some powers of
+    // two above the largest value loses nothing.
+    // (With the residuals of bf16_residual and without the clamps of the anchor
+    // factors, which the exact form makes needless: 417 of 4502 VALU
+    // instructions less; 8192 tokens on 32 heads 285.8 -> 273.8 us in all.)
+    int ksh, qsh, aqsh;
+    float kel1;
+    {
+        auto max4_bf16 = [](const uint32_t *p) {
+            const uint4 u = *reinterpret_cast<const uint4 *>(p);
+            return __uint_as_float(max(max(u.x, u.y), max(u.z, u.w)) << 16);
+        };
+        const float km = norm ? 1.f : max4_bf16(sm.kmax);
+        const float qm = (norm ? 1.f : max4_bf16(sm.qmax)) * fabsf(a.scale);
+        const int up = static_cast<int>(
+            fminf(ceilf(static_cast<float>(BT) * max4_mag(*reinterpret_cast<const float4 *>(sm.grow))), 100.f));
+        const int sk = f16_shift(km);
+        const int sq = f16_shift(qm);
+        ksh = __builtin_amdgcn_readfirstlane(sk - up);
+        qsh = __builtin_amdgcn_readfirstlane(sq - up);
+        // max|k| < 2^(14 - sk), max|q| < 2^(14 - sq): 128 of their products stay
+        // below 2^14 under 2^(sk + sq - 21); normalized rows' below max|q|
+        aqsh = __builtin_amdgcn_readfirstlane((norm ? sq : max(min(sk + sq - 21, 120), -120)) - up);
+        kel1 = ldexpf(128.f * km, up);
+    }
 
     // 8 channels {32s + kperm(gq, e)} of one row: two 16-byte reads each
     // from the (normalized) k and the cumsum tiles.
@@ -964,17 +1032,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         // factor e^(anchor - G_j) at most 8 (diagonal block, j > anchor) and
         // is e^(<=0) for every earlier block, so fp32 and bf16 hold both while
         // 8 consecutive tokens decay by less than 2^kMaxExp2 (about 87 nat).
-        // Beyond that the exponents are clamped: results stay finite but are
-        // no longer exact (the precondition stated with the C ABI).
+        // Beyond that the products may not be finite; the exact form replaces
+        // every one of them.
         float anc[2][8];
 #pragma unroll
         for (int sl = 0; sl < 2; ++sl) {
             load_g8(16 * I + kAnchorRow, 2 * sh + sl, anc[sl]);
         }
         bf16x8 Rh[2], Rl[2], Qh[2], Ql[2];
-        float qg[2][8];  // q e^G of this half's two slices: one record scale
-        float ke[2][8];  // e^G k of the same rows and channels: one record scale
-        float l1 = 0.f;  // this lane's share of the row's sum of |e^G k| over the half
+        float qg[2][8];  // q e^G of this half's two slices
+        float ke[2][8];  // e^G k of the same rows and channels
 #pragma unroll
         for (int sl = 0; sl < 2; ++sl) {
             const int s = 2 * sh + sl;
@@ -983,31 +1050,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             load_g8(ri, s, gg);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float ex = ex2(fminf(gg[e] - anc[sl][e], kMaxExp2));
+                const float ex = ex2(gg[e] - anc[sl][e]);
                 const float eg = ex2(gg[e]);
                 const float qn = qv[sl][e] * qscale;
                 rv[e] = kk[e] * ex;
                 qa[e] = qn * ex;
                 qg[sl][e] = qn * eg;
                 ke[sl][e] = kk[e] * eg;
-                l1 += fabsf(ke[sl][e]);
             }
             split_bf16x8(rv, Rh[sl], Rl[sl]);
             split_bf16x8(qa, Qh[sl], Ql[sl]);
         }
-        float *sc = reinterpret_cast<float *>(rec + kOffSc);
-        store_frags_f16<2>(rec, kOffQg, I * 4 + 2 * sh, sc + kScQg + I * 4 + 2 * sh, lane, qg, 2);
+        store_frags_f16<2>(rec, kOffQg, I * 4 + 2 * sh, qsh, lane, qg);
         // e^G k: the A fragments of row tile I, slices 2sh and 2sh+1, for the
-        // scan's (e^G k) S; and this half's max over the tile's rows of
-        // sum_k |e^G k|, which the scan adds to the other half's to bound that
-        // product with max |S|
-        store_frags_f16<2>(rec, kOffKe, I * 4 + 2 * sh, sc + kScKe + I * 4 + 2 * sh, lane, ke, 2);
-        l1 += __shfl_xor(l1, 16);
-        l1 += __shfl_xor(l1, 32);
-        l1 = wave_max_mag(l1);
-        if (lane == 0) {
-            sc[kScKel1 + 4 * sh + I] = l1;
-        }
+        // scan's (e^G k) S
+        store_frags_f16<2>(rec, kOffKe, I * 4 + 2 * sh, ksh, lane, ke);
         // pairs (I, J), J <= I, over this half's channels
 #pragma unroll
         for (int J = 0; J < (ii == 0 ? 4 : 2); ++J) {
@@ -1023,13 +1080,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 float kk[8], gg[8], cv[8];
                 load_k8(rj, s, kk);
                 load_g8(rj, s, gg);
-                // blocks 0 and 1 against the upper row block I = IA >= 2 are
-                // earlier blocks: anchor - G_j <= 0 (g <= 0), no clamp needed
-                const bool earlier = ii == 0 && J < 2;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const float d = anc[sl][e] - gg[e];
-                    cv[e] = kk[e] * ex2(earlier ? d : fminf(d, kMaxExp2));
+                    cv[e] = kk[e] * ex2(anc[sl][e] - gg[e]);
                 }
                 bf16x8 Ch, Cl;
                 split_bf16x8(cv, Ch, Cl);
@@ -1060,28 +1113,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     };
     // kd[t][16mk + r] = k_t e^(G_last - G_t) for the rows t = 32s + kperm(gq, e)
-    // (B fragments of T^T kd, mk = 2 wave + tt), fp16 hi + lo with one
-    // power-of-two scale 2^-shift per mk; S6 uses them from registers.
+    // (B fragments of T^T kd, mk = 2 wave + tt), fp16 hi + lo scaled by 2^ksh;
+    // S6 uses them from registers.
     u32x4 kdh[2][2], kdl[2][2];
-    int kdsh[2];
-    auto to_frags = [&](const float (&x)[2][8], u32x4 (&fh)[2], u32x4 (&fl)[2], int &shift) {
-        float m = 0.f;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                m = fmaxf(m, fabsf(x[s][e]));
-            }
-        }
-        const int sh = f16_shift(wave_max_mag(m));
+    auto to_frags = [&](const float (&x)[2][8], u32x4 (&fh)[2], u32x4 (&fl)[2], int shift) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
             f16x8 hi, lo;
-            split_f16x8(x[s], sh, hi, lo);
+            split_f16x8(x[s], shift, hi, lo);
             fh[s] = as_u32x4(hi);
             fl[s] = as_u32x4(lo);
         }
-        shift = sh;
     };
 #pragma unroll
     for (int tt = 0; tt < 2; ++tt) {
@@ -1099,7 +1141,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 x[s][e] = kr[e] * ex2(gl - sm.u.early.G[t][k]);
             }
         }
-        to_frags(x, kdh[tt], kdl[tt], kdsh[tt]);
+        to_frags(x, kdh[tt], kdl[tt], ksh);
     }
     if (tid < DK) {
         reinterpret_cast<float *>(rec + kOffGl)[tid] = ex2(sm.u.early.G[BT - 1][tid]);
@@ -1111,7 +1153,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     bool tracked = false;
     char *tr = nullptr;
     u32x4 kth[2][2], ktl[2][2];
-    int ktsh[2] = {0, 0};
     if (a.track_indices != nullptr) {
         const int ts = a.track_indices[n];
         const int tl = a.track_lens[n];
@@ -1135,7 +1176,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         x[s][e] = t < rr ? kr[e] * ex2(gr - sm.u.early.G[t][k]) : 0.f;
                     }
                 }
-                to_frags(x, kth[tt], ktl[tt], ktsh[tt]);
+                to_frags(x, kth[tt], ktl[tt], ksh);
             }
             if (tid < DK) {
                 reinterpret_cast<float *>(tr + kTrOffGl)[tid] = ex2(sm.u.early.G[rr - 1][tid]);
@@ -1353,6 +1394,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // result tiles over token rows [32s, 32s+16) and [32s+16, 32s+32) is the
     // A fragment of token slice s.
     float *sc = reinterpret_cast<float *>(rec + kOffSc);
+    if (tid == 0) {
+        sc[kScKe] = ldexpf(1.f, -ksh);
+        sc[kScQg] = ldexpf(1.f, -qsh);
+        sc[kScKel1] = kel1;
+    }
     {
         // T^T fragments of row tile tt = wave (both token slices): lane (r, g)
         // element e holds T[32s + kperm(g, e)][16 wave + r] (zero where the
@@ -1421,7 +1467,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int mk = 2 * wave + tt;
         float x[2][8];
         int ex[4];
-        ttb(kdh[tt], kdl[tt], kdsh[tt], x, 3, ex);
+        ttb(kdh[tt], kdl[tt], ksh, x, 3, ex);
         store_frags_f16_exp<2>(rec, kOffKd, mk * 2, sc + kScKd + mk, lane, x, ex);
     }
     if (tracked) {
@@ -1430,7 +1476,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int mk = 2 * wave + tt;
             float x[2][8];
             int ex[4];
-            ttb(kth[tt], ktl[tt], ktsh[tt], x, 3, ex);
+            ttb(kth[tt], ktl[tt], ksh, x, 3, ex);
             store_frags_f16_exp<2>(tr, kTrOffKd, mk * 2, reinterpret_cast<float *>(tr + kTrOffSc) + mk, lane, x,
                                    ex);
         }
@@ -1453,7 +1499,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             }
         }
         u32x4 aqh[2], aql[2];
-        int aqsh;
         to_frags(ax, aqh, aql, aqsh);
         float x[2][8];
 #pragma unroll
@@ -1943,8 +1988,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
         struct OpsB {
             f16x8 Kef[4];
             f32x4 vv[NT];
-            float4 kesc;
-            float vmax, kel1;
+            float kesc, vmax, kel1;
         };
         auto read_b = [&](OpsB &op, int p) {
             const char *st = sm.stg[p];
@@ -1972,8 +2016,8 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
             }
             const float4 um = *reinterpret_cast<const float4 *>(&sm.vmax[p][0]);
             op.vmax = max4_mag(um);
-            op.kesc = *reinterpret_cast<const float4 *>(sc + kScKe + 4 * wr);
-            op.kel1 = kel1_bound(sc);
+            op.kesc = sc[kScKe];
+            op.kel1 = sc[kScKel1];
         };
         // chunk j (of the item, PERS) in the stage of parity p
         auto step = [&](int j, int p, const OpsG &og, OpsG &next) {
@@ -2028,7 +2072,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
             const float4 ss = *reinterpret_cast<const float4 *>(&sm.sscale[p][0]);
             const int sv = f16_shift(ob.vmax + ob.kel1 * max4_mag(sx));
             const float inv_v = ldexpf(1.f, -sv);
-            const float fw[4] = {ob.kesc.x * ss.x, ob.kesc.y * ss.y, ob.kesc.z * ss.z, ob.kesc.w * ss.w};
+            const float fw[4] = {ob.kesc * ss.x, ob.kesc * ss.y, ob.kesc * ss.z, ob.kesc * ss.w};
             f16x8 Kd[2][2];
             f32x4 gl[2];
             float2 kdsc;
@@ -2333,7 +2377,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
         struct OpsO {
             f16x8 Qg[4];
             f16x8 Aq[2];
-            float4 qsc;
+            float qsc;
         };
         Cur cl;  // PERS: load_out's position (one chunk ahead)
         Cur co;  // PERS: finish's position (one chunk behind)
@@ -2352,7 +2396,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
                 op.Aq[0] = as_f16x8(aq[aq_frag(wr, 0) * 64 + lane]);
                 op.Aq[1] = as_f16x8(aq[aq_frag(wr, wr >= 2 ? 1 : 0) * 64 + lane]);
             }
-            op.qsc = *reinterpret_cast<const float4 *>(rec + kOffSc + 4 * (kScQg + 4 * wr));
+            op.qsc = *reinterpret_cast<const float *>(rec + kOffSc + 4 * kScQg);
         };
         auto aqk_y = [&](const OpsO &op, int j) {
             const int p = j & 1;
@@ -2360,7 +2404,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
             const float *sc = reinterpret_cast<const float *>(st + St::kMisc) + DK;
             const float4 um = *reinterpret_cast<const float4 *>(&sm.vmax[p][0]);
             const float4 sx = *reinterpret_cast<const float4 *>(&sm.smax[p][0]);
-            const int sv = f16_shift(max4_mag(um) + kel1_bound(sc) * max4_mag(sx));
+            const int sv = f16_shift(max4_mag(um) + sc[kScKel1] * max4_mag(sx));
             const float f = sc[kScAq + wr] * ldexpf(1.f, -sv);
             // rows [16wr, 16wr+16) meet tokens >= 32 only for wr >= 2
             const f16x8 aq0 = LEAN ? op.Aq[0] : stage_frag(st, kStAq + aq_frag(wr, 0), lane);
@@ -2465,7 +2509,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
             }
             f32x4 Pn[NT];
             const float4 ss = *reinterpret_cast<const float4 *>(&sm.sscale[p][0]);
-            const float fq[4] = {cur.qsc.x * ss.x, cur.qsc.y * ss.y, cur.qsc.z * ss.z, cur.qsc.w * ss.w};
+            const float fq[4] = {cur.qsc * ss.x, cur.qsc * ss.y, cur.qsc * ss.z, cur.qsc * ss.w};
 #pragma unroll
             for (int ct = 0; ct < NT; ++ct) {
                 f32x4 acc[4];
