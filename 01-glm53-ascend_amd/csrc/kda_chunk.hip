@@ -572,6 +572,59 @@ __device__ __forceinline__ uint32_t keep_mask(bool keep) {
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
+// The right-looking inverse of unit lower triangular 16x16 blocks L, one per
+// 16-lane row: acc (the identity's column) becomes the inverse's, in steps
+// j = 0 .. 14 of acc[i] -= L[i][j] acc[j], i > j. lt[i] of lane j of the row is
+// L[i][j], which v_fmac_f32's DPP row_newbcast:j gives to every lane: 120
+// instructions and no LDS access. (As C++ each takes a v_mov_b32_dpp and a
+// multiply-add.) One asm block, so nothing writes lt between the wait states
+// a DPP operand needs (the s_nop) and its uses.
+__device__ __forceinline__ void invert_blocks(const float (&lt)[16], float (&acc)[16]) {
+#define KDA_F(i, j) \
+    "v_fmac_f32_dpp %[a" #i "], -%[l" #i "], %[a" #j "] row_newbcast:" #j " row_mask:0xf bank_mask:0xf\n\t"
+#define KDA_F15(j) KDA_F(15, j)
+#define KDA_F14(j) KDA_F(14, j) KDA_F15(j)
+#define KDA_F13(j) KDA_F(13, j) KDA_F14(j)
+#define KDA_F12(j) KDA_F(12, j) KDA_F13(j)
+#define KDA_F11(j) KDA_F(11, j) KDA_F12(j)
+#define KDA_F10(j) KDA_F(10, j) KDA_F11(j)
+#define KDA_F9(j) KDA_F(9, j) KDA_F10(j)
+#define KDA_F8(j) KDA_F(8, j) KDA_F9(j)
+#define KDA_F7(j) KDA_F(7, j) KDA_F8(j)
+#define KDA_F6(j) KDA_F(6, j) KDA_F7(j)
+#define KDA_F5(j) KDA_F(5, j) KDA_F6(j)
+#define KDA_F4(j) KDA_F(4, j) KDA_F5(j)
+#define KDA_F3(j) KDA_F(3, j) KDA_F4(j)
+#define KDA_F2(j) KDA_F(2, j) KDA_F3(j)
+#define KDA_F1(j) KDA_F(1, j) KDA_F2(j)
+    asm("s_nop 1\n\t"
+        KDA_F1(0) KDA_F2(1) KDA_F3(2) KDA_F4(3) KDA_F5(4) KDA_F6(5) KDA_F7(6) KDA_F8(7)
+        KDA_F9(8) KDA_F10(9) KDA_F11(10) KDA_F12(11) KDA_F13(12) KDA_F14(13) KDA_F15(14)
+        : [a0] "+v"(acc[0]), [a1] "+v"(acc[1]), [a2] "+v"(acc[2]), [a3] "+v"(acc[3]), [a4] "+v"(acc[4]),
+          [a5] "+v"(acc[5]), [a6] "+v"(acc[6]), [a7] "+v"(acc[7]), [a8] "+v"(acc[8]), [a9] "+v"(acc[9]),
+          [a10] "+v"(acc[10]), [a11] "+v"(acc[11]), [a12] "+v"(acc[12]), [a13] "+v"(acc[13]), [a14] "+v"(acc[14]),
+          [a15] "+v"(acc[15])
+        : [l1] "v"(lt[1]), [l2] "v"(lt[2]), [l3] "v"(lt[3]), [l4] "v"(lt[4]), [l5] "v"(lt[5]), [l6] "v"(lt[6]),
+          [l7] "v"(lt[7]), [l8] "v"(lt[8]), [l9] "v"(lt[9]), [l10] "v"(lt[10]), [l11] "v"(lt[11]),
+          [l12] "v"(lt[12]), [l13] "v"(lt[13]), [l14] "v"(lt[14]), [l15] "v"(lt[15]));
+#undef KDA_F
+#undef KDA_F1
+#undef KDA_F2
+#undef KDA_F3
+#undef KDA_F4
+#undef KDA_F5
+#undef KDA_F6
+#undef KDA_F7
+#undef KDA_F8
+#undef KDA_F9
+#undef KDA_F10
+#undef KDA_F11
+#undef KDA_F12
+#undef KDA_F13
+#undef KDA_F14
+#undef KDA_F15
+}
+
 struct PrepShared {
     union {
         struct {
@@ -584,8 +637,14 @@ struct PrepShared {
             // Strict upper triangle: L^T, LT[j][i] = beta_i Akk[i][j] (j < i).
             // Lower triangle with the diagonal: Aqk[i][j] (j <= i).
             float LT[BT][kPadX];
-            u32x4 TT[4][2][2][64];  // T^T A fragments (row tile, token slice, hi / lo) (S6)
-            int ttsh[4];            // their power-of-two shift per row tile
+            union {
+                f32x4 part[4][5][64];  // S3's partial products on their way to the other half's wave
+                float M[4][16][20];    // the inverse's intermediate tiles (S5), rows padded
+                struct {
+                    u32x4 TT[4][2][2][64];  // T^T A fragments (row tile, token slice, hi / lo) (S6)
+                    int ttsh[4];            // their power-of-two shift per row tile
+                };
+            };
         } mid;
     } u;
     float beta[BT];
@@ -665,7 +724,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // a scalar: roles branch without masks
     const int r = lane & 15;
     const int gq = lane >> 4;
     char *rec = ws + LY.recs + (static_cast<size_t>(c % ring) * H + h) * kRecBytes;
@@ -1235,157 +1294,192 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 
     lds_barrier();  // G and K are dead from here on
-    // S3's two channel halves meet in LT, which lies over the dead G: half
-    // sh = 1 stores its partial products, then half sh = 0 adds its own and
-    // applies beta. Every LT element is written: block (J, I), J < I, holds
-    // Akk^T; block (I, J), J < I, holds Aqk; a diagonal block holds Akk^T
-    // above and Aqk on and below its diagonal.
-    if (sh == 1) {
-#pragma unroll
-        for (int ii = 0; ii < 2; ++ii) {
-            const int I = ii == 0 ? IA : 3 - IA;
-#pragma unroll
-            for (int J = 0; J < (ii == 0 ? 4 : 2); ++J) {
-                if (J > I) {
-                    break;
-                }
-                if (J < I) {
-                    *reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * J + r][16 * I + 4 * gq]) = pk[ii][J];
-                    *reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * I + r][16 * J + 4 * gq]) = pq[ii][J];
-                } else {
-                    f32x4 m;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        m[e] = r < 4 * gq + e ? pk[ii][J][e] : pq[ii][J][e];
-                    }
-                    *reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * I + r][16 * I + 4 * gq]) = m;
-                }
-            }
+    // S3's two channel halves meet: of a wave pair's ten tiles (Akk and Aqk of
+    // its three pairs off the diagonal and two on it) half 0 sums the diagonal
+    // ones and the first, half 1 the other five, each leaving the other its own
+    // partials in LDS. Every LT element is written: block (J, I), J < I, holds
+    // beta Akk^T; block (I, J), J < I, Aqk; a diagonal block beta Akk^T above
+    // and Aqk on and below its diagonal.
+    const bool upper = wave < 2;  // row blocks 3 and 0, else 2 and 1
+    // off-diagonal pair f of this wave: (3,0) (3,1) (3,2), or (2,0) (2,1) (1,0)
+    auto off_k = [&](int f) -> const f32x4 & { return f < 2 || upper ? pk[0][f] : pk[1][0]; };
+    auto off_q = [&](int f) -> const f32x4 & { return f < 2 || upper ? pq[0][f] : pq[1][0]; };
+    const f32x4 dk0 = upper ? pk[0][3] : pk[0][2], dq0 = upper ? pq[0][3] : pq[0][2];  // (IA, IA)
+    const f32x4 dk1 = upper ? pk[1][0] : pk[1][1], dq1 = upper ? pq[1][0] : pq[1][1];  // (3 - IA, 3 - IA)
+    {
+        f32x4(&mine)[5][64] = sm.u.mid.part[wave];
+        if (sh == 0) {
+            mine[0][lane] = off_q(0);
+            mine[1][lane] = off_k(1);
+            mine[2][lane] = off_q(1);
+            mine[3][lane] = off_k(2);
+            mine[4][lane] = off_q(2);
+        } else {
+            mine[0][lane] = dk0;
+            mine[1][lane] = dq0;
+            mine[2][lane] = dk1;
+            mine[3][lane] = dq1;
+            mine[4][lane] = off_k(0);
         }
     }
-    // X: the six upper 16x16 blocks (I, J > I) zero, one float4 per store
-    for (int f = tid; f < 6 * 64; f += kThreads) {
-        const int blk = f >> 6;                      // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
-        const int bi = blk < 3 ? 0 : (blk < 5 ? 1 : 2);
-        const int bj = blk < 3 ? blk + 1 : (blk < 5 ? blk - 1 : 3);
-        const int row = (f & 63) >> 2;
-        *reinterpret_cast<float4 *>(&sm.u.mid.X[16 * bi + row][16 * bj + 4 * (f & 3)]) =
-            make_float4(0.f, 0.f, 0.f, 0.f);
-    }
     lds_barrier();
-    if (sh == 0) {
-#pragma unroll
-        for (int ii = 0; ii < 2; ++ii) {
-            const int I = ii == 0 ? IA : 3 - IA;
+    {
+        const f32x4(&other)[5][64] = sm.u.mid.part[wave ^ 1];
+        auto put_k = [&](int I, int J, const f32x4 &x) {
             const float4 b4 = *reinterpret_cast<const float4 *>(&sm.beta[16 * I + 4 * gq]);
-            const f32x4 bv = {b4.x, b4.y, b4.z, b4.w};
+            *reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * J + r][16 * I + 4 * gq]) = x * f32x4{b4.x, b4.y, b4.z, b4.w};
+        };
+        auto put_q = [&](int I, int J, const f32x4 &x) {
+            *reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * I + r][16 * J + 4 * gq]) = x;
+        };
+        auto put_diag = [&](int I, const f32x4 &k, const f32x4 &q) {
+            const float4 b4 = *reinterpret_cast<const float4 *>(&sm.beta[16 * I + 4 * gq]);
+            const f32x4 xk = k * f32x4{b4.x, b4.y, b4.z, b4.w};
+            f32x4 m;
 #pragma unroll
-            for (int J = 0; J < (ii == 0 ? 4 : 2); ++J) {
-                if (J > I) {
-                    break;
-                }
-                if (J < I) {
-                    f32x4 *pa = reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * J + r][16 * I + 4 * gq]);
-                    f32x4 *pb = reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * I + r][16 * J + 4 * gq]);
-                    const f32x4 xa = *pa;
-                    const f32x4 xb = *pb;
-                    *pa = (xa + pk[ii][J]) * bv;
-                    *pb = xb + pq[ii][J];
-                } else {
-                    f32x4 *pd = reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * I + r][16 * I + 4 * gq]);
-                    const f32x4 xd = *pd;
-                    f32x4 m;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        m[e] = r < 4 * gq + e ? (xd[e] + pk[ii][J][e]) * bv[e] : xd[e] + pq[ii][J][e];
-                    }
-                    *pd = m;
-                }
+            for (int e = 0; e < 4; ++e) {
+                m[e] = r < 4 * gq + e ? xk[e] : q[e];
             }
+            *reinterpret_cast<f32x4 *>(&sm.u.mid.LT[16 * I + r][16 * I + 4 * gq]) = m;
+        };
+        const int I2 = upper ? 3 : 1;  // the third off-diagonal pair (I2, J2)
+        const int J2 = upper ? 2 : 0;
+        if (sh == 0) {
+            put_diag(IA, dk0 + other[0][lane], dq0 + other[1][lane]);
+            put_diag(3 - IA, dk1 + other[2][lane], dq1 + other[3][lane]);
+            put_k(IA, 0, off_k(0) + other[4][lane]);
+        } else {
+            put_q(IA, 0, other[0][lane] + off_q(0));
+            put_k(IA, 1, other[1][lane] + off_k(1));
+            put_q(IA, 1, other[2][lane] + off_q(1));
+            put_k(I2, J2, other[3][lane] + off_k(2));
+            put_q(I2, J2, other[4][lane] + off_q(2));
         }
     }
     lds_barrier();
 
     // ---- S5: X = (I + L)^-1 (blocked, fp32); T = X diag(beta) is formed as S6 reads X
-    // Diagonal 16x16 blocks, right-looking: column c of block w per lane c.
-    if (lane < 16) {
-        const int b0 = 16 * wave;
-        const int col = lane;
-        // Constant loop bounds with a compile-time i > j mask: every acc[]
-        // index is static, so the array stays in registers (a bound that
-        // depends on j leaves the inner loop rolled and turns acc[] into a
-        // runtime-indexed select chain).
-        float acc[16];
+    // A serial stretch, so what counts is its length: with the hand-over above
+    // and S6's Aqk fragments taken into the diagonal blocks' shadow a workgroup
+    // went from 34,200 clocks to 30,000 (8192 tokens, 32 heads: 274 -> 263 us;
+    // before, half 0 summed all tiles, every wave formed one diagonal block from
+    // LDS broadcasts, 2050 clocks against 1500, and the rest took three levels).
+    if (wave == 0) {
+        // The four diagonal 16x16 blocks at once, right-looking: lane (c, g)
+        // forms column c of block g. Lane j of a 16-lane row holds row j of its
+        // block of LT, so L[i][j] comes to all columns as a DPP broadcast of
+        // lane j within the row.
+        float lt[16], acc[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            acc[i] = i == col ? 1.f : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < 15; ++j) {
-            const float xj = acc[j];
-            float lrow[16];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float4 t4 = *reinterpret_cast<const float4 *>(&sm.u.mid.LT[b0 + j][b0 + 4 * q]);
-                lrow[4 * q + 0] = t4.x;
-                lrow[4 * q + 1] = t4.y;
-                lrow[4 * q + 2] = t4.z;
-                lrow[4 * q + 3] = t4.w;
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                if (i > j) {
-                    acc[i] -= lrow[i] * xj;
-                }
-            }
+        for (int q = 0; q < 4; ++q) {
+            const float4 t4 = *reinterpret_cast<const float4 *>(&sm.u.mid.LT[16 * gq + r][16 * gq + 4 * q]);
+            lt[4 * q + 0] = t4.x;
+            lt[4 * q + 1] = t4.y;
+            lt[4 * q + 2] = t4.z;
+            lt[4 * q + 3] = t4.w;
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            sm.u.mid.X[b0 + i][b0 + col] = acc[i];
+            acc[i] = i == r ? 1.f : 0.f;
         }
+        invert_blocks(lt, acc);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            sm.u.mid.X[16 * gq + i][16 * gq + r] = acc[i];
+        }
+    } else {
+        // X's six upper 16x16 blocks (I, J > I) are zero, one float4 per store
+        for (int f = tid - 64; f < 6 * 64; f += kThreads - 64) {
+            const int blk = f >> 6;  // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
+            const int bi = blk < 3 ? 0 : (blk < 5 ? 1 : 2);
+            const int bj = blk < 3 ? blk + 1 : (blk < 5 ? blk - 1 : 3);
+            const int row = (f & 63) >> 2;
+            *reinterpret_cast<float4 *>(&sm.u.mid.X[16 * bi + row][16 * bj + 4 * (f & 3)]) =
+                make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    // B = Aqk^T of row tile mt = wave for S6, fp16 hi + lo: lane (r, g) element e
+    // = Aqk[16 wave + r][32s + kperm(g, e)] (zero above the diagonal). Here, since
+    // three of the four waves wait for the diagonal blocks.
+    u32x4 aqh[2], aql[2];
+    {
+        const int row = 16 * wave + r;
+        float ax[2][8];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const float4 x0 = *reinterpret_cast<const float4 *>(&sm.u.mid.LT[row][32 * s + 4 * gq]);
+            const float4 x1 = *reinterpret_cast<const float4 *>(&sm.u.mid.LT[row][32 * s + 16 + 4 * gq]);
+            const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                ax[s][e] = 32 * s + kperm(gq, e) <= row ? xv[e] : 0.f;
+            }
+        }
+        to_frags(ax, aqh, aql, aqsh);
     }
     lds_barrier();
-    // Off-diagonal blocks by level d = I - J, one (I, J) per wave (wave J),
-    // on the fp32 MFMA (v_mfma_f32_16x16x4_f32: lane (r, g) supplies A[r][g]
-    // and B[g][r] of each 4-wide K step; C as for the bf16 tiles):
-    //   M_IJ = sum_{K=J}^{I-1} L_IK X_KJ,   X_IJ = -X_II M_IJ.
-    // M_IJ passes through the wave's still-zero upper block (J, I) of X, which
-    // is cleared again before the level's barrier.
-    for (int d = 1; d < 4; ++d) {
-        const int J = wave;
-        const int I = J + d;
-        if (I < 4) {
-            f32x4 m = {0.f, 0.f, 0.f, 0.f};
-            for (int K = J; K < I; ++K) {
+    // Off the diagonal by halves, on the fp32 MFMA (v_mfma_f32_16x16x4_f32: lane
+    // (r, g) supplies A[r][g] and B[g][r] of each 4-wide K step; C as for the
+    // bf16 tiles). First the 32x32 diagonal blocks' lower tiles, wave 0 (1, 0)
+    // and wave 1 (3, 2): X_IJ = -X_II (L_IJ X_JJ); then the lower left 32x32
+    // block, a tile (I, J) per wave: M_IJ = sum_K L_IK X_KJ over the upper half's
+    // K, X_IJ = -sum_K X_IK M_KJ over the lower half's. The intermediate tiles
+    // pass through LDS.
+    // c + L_IK X_KJ, and c + X_IK m (m: a tile in LDS)
+    auto mul_lx = [&](int I, int K, int J, f32x4 c) {
 #pragma unroll
-                for (int k4 = 0; k4 < 4; ++k4) {
-                    const int kk = 16 * K + 4 * k4 + gq;
-                    m = __builtin_amdgcn_mfma_f32_16x16x4f32(sm.u.mid.LT[kk][16 * I + r],
-                                                            sm.u.mid.X[kk][16 * J + r], m, 0, 0, 0);
-                }
-            }
-            // lane (r, gq) holds M[4gq + i][r]; park it row-major in block (J, I)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sm.u.mid.X[16 * J + 4 * gq + i][16 * I + r] = m[i];
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            f32x4 x = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int k4 = 0; k4 < 4; ++k4) {
-                x = __builtin_amdgcn_mfma_f32_16x16x4f32(sm.u.mid.X[16 * I + r][16 * I + 4 * k4 + gq],
-                                                        sm.u.mid.X[16 * J + 4 * k4 + gq][16 * I + r], x,
-                                                        0, 0, 0);
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                sm.u.mid.X[16 * I + 4 * gq + i][16 * J + r] = -x[i];
-                sm.u.mid.X[16 * J + 4 * gq + i][16 * I + r] = 0.f;
-            }
+        for (int k4 = 0; k4 < 4; ++k4) {
+            const int kk = 16 * K + 4 * k4 + gq;
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(sm.u.mid.LT[kk][16 * I + r], sm.u.mid.X[kk][16 * J + r], c, 0, 0,
+                                                    0);
         }
-        lds_barrier();
+        return c;
+    };
+    auto mul_xm = [&](int I, int K, const float (&m)[16][20], f32x4 c) {
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4) {
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(sm.u.mid.X[16 * I + r][16 * K + 4 * k4 + gq], m[4 * k4 + gq][r],
+                                                    c, 0, 0, 0);
+        }
+        return c;
+    };
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    // lane (r, gq) holds x[4gq + i][r]
+    auto put_m = [&](float (&m)[16][20], const f32x4 &x) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            m[4 * gq + i][r] = x[i];
+        }
+    };
+    auto put_x = [&](int I, int J, const f32x4 &x) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            sm.u.mid.X[16 * I + 4 * gq + i][16 * J + r] = -x[i];
+        }
+    };
+    if (wave < 2) {
+        const int J = 2 * wave;
+        put_m(sm.u.mid.M[wave], mul_lx(J + 1, J, J, zero4));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        put_x(J + 1, J, mul_xm(J + 1, J + 1, sm.u.mid.M[wave], zero4));
     }
+    lds_barrier();
+    {
+        const int I = 2 + (wave >> 1);
+        const int J = wave & 1;
+        f32x4 m = mul_lx(I, 1, J, zero4);
+        if (J == 0) {
+            m = mul_lx(I, 0, 0, m);
+        }
+        put_m(sm.u.mid.M[wave], m);
+        lds_barrier();
+        f32x4 x = mul_xm(I, I, sm.u.mid.M[wave], zero4);
+        if (I == 3) {
+            x = mul_xm(3, 2, sm.u.mid.M[J], x);
+        }
+        put_x(I, J, x);
+    }
+    lds_barrier();
 
     // ---- S6: T^T kd and Aqk T, T = X diag(beta) --------------------------------
     // The scan never forms u = T v or w = T (e^G k): with y = v - (e^G k) S,
@@ -1482,24 +1576,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     }
     {
-        // (Aqk T) fragments of row tile mt = wave: B = Aqk^T, lane (r, g)
-        // element e = Aqk[16 wave + r][32s + kperm(g, e)] (zero above the
-        // diagonal); tokens after the row's last contribute nothing, so only
-        // the tiles tt <= wave are formed and slice 1 only for wave >= 2
-        const int row = 16 * wave + r;
-        float ax[2][8];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const float4 x0 = *reinterpret_cast<const float4 *>(&sm.u.mid.LT[row][32 * s + 4 * gq]);
-            const float4 x1 = *reinterpret_cast<const float4 *>(&sm.u.mid.LT[row][32 * s + 16 + 4 * gq]);
-            const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                ax[s][e] = 32 * s + kperm(gq, e) <= row ? xv[e] : 0.f;
-            }
-        }
-        u32x4 aqh[2], aql[2];
-        to_frags(ax, aqh, aql, aqsh);
+        // (Aqk T) fragments of row tile mt = wave; tokens after the row's last
+        // contribute nothing, so only the tiles tt <= wave are formed and slice 1
+        // only for wave >= 2
         float x[2][8];
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
