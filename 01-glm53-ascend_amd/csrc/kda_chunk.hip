@@ -73,6 +73,8 @@
 namespace kda {
 namespace chunk {
 
+using ChunkLaunch = Launch<KdaChunkArgs>;
+
 constexpr int BT = 64;   // tokens per chunk
 constexpr int DK = 128;  // K == V
 constexpr int kThreads = 256;
@@ -350,10 +352,10 @@ __device__ __forceinline__ void store_frags_f16_exp(char *base, int off, int idx
 }
 
 
-__device__ __forceinline__ void seq_bounds(const KdaChunkArgs &a, int n, int &bos, int &eos) {
+__device__ __forceinline__ void seq_bounds(const ChunkLaunch &a, int n, int &bos, int &eos) {
     const int T = a.num_tokens;
-    bos = a.cu_seqlens[n];
-    eos = a.cu_seqlens[n + 1];
+    bos = a.cu(n);
+    eos = a.cu(n + 1);
     bos = bos < 0 ? 0 : (bos > T ? T : bos);
     eos = eos < bos ? bos : (eos > T ? T : eos);
 }
@@ -373,7 +375,7 @@ __device__ __forceinline__ void seq_bounds(const KdaChunkArgs &a, int n, int &bo
 constexpr int kPersMaxSeqs = 4096;
 constexpr int kPersMaxItems = 256;
 
-__global__ __launch_bounds__(1024) void chunk_index_kernel(const KdaChunkArgs a, int *cs, int4 *sched, int sort) {
+__global__ __launch_bounds__(1024) void chunk_index_kernel(const ChunkLaunch a, int *cs, int4 *sched, int sort) {
     // With the schedule, every per-sequence value is loaded once, up front,
     // into LDS, so the sort and the table wait on no global round trip.
     __shared__ int part[16];                            // each wave's chunk total
@@ -396,15 +398,15 @@ __global__ __launch_bounds__(1024) void chunk_index_kernel(const KdaChunkArgs a,
         const int c = (eos - bos + BT - 1) / BT;
         sum += c;
         if (dosort) {
-            int slot = a.state_indices[n];
+            int slot = a.slot_index(n);
             if (slot < 0 || static_cast<int64_t>(slot) >= a.num_slots) {
                 slot = 0;
             }
             int tslot = 0;
             int tlen = -1;
             if (track) {
-                tslot = a.track_indices[n];
-                const int tl = a.track_lens[n];
+                tslot = a.track_index(n);
+                const int tl = a.track_length(n);
                 if (tslot <= 0 || static_cast<int64_t>(tslot) >= a.num_slots) {
                     tslot = 0;
                 } else {
@@ -669,7 +671,7 @@ static_assert(sizeof(PrepShared) <= 80 * 1024, "two prepare workgroups per CU");
 // since the affine form's first pass scans all segments at once.
 template <int GATE>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void chunk_prepare_kernel(
-    const KdaChunkArgs a, char *ws, int ring, int c_lo, int c_hi, int seg_w) {
+    const ChunkLaunch a, char *ws, int ring, int c_lo, int c_hi, int seg_w) {
     __shared__ PrepShared sm;
     // Workgroups run chunk-descending, heads fastest: the scan starts with the
     // first chunk of every sequence and head, so those records are written
@@ -1213,8 +1215,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     char *tr = nullptr;
     u32x4 kth[2][2], ktl[2][2];
     if (a.track_indices != nullptr) {
-        const int ts = a.track_indices[n];
-        const int tl = a.track_lens[n];
+        const int ts = a.track_index(n);
+        const int tl = a.track_length(n);
         const int rr = tl - BT * jc;
         if (ts > 0 && static_cast<int64_t>(ts) < a.num_slots && rr > 0 && rr < len) {
             tracked = true;
@@ -1726,7 +1728,7 @@ __device__ __forceinline__ f16x8 stage_frag(const char *st, int f, int lane) {
 // workgroup per item paid at its start (about 3.9 us: dispatch, the first
 // loads, the pipeline's fill and drain) is paid once per workgroup.
 template <int NT, bool SEG, bool AFF = false, bool PERS = false>
-__global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunkArgs a, const char *ws,
+__global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLaunch a, const char *ws,
                                                                   int ring, int s_lo, int s_hi) {
     // the affine first pass runs the lean form (its chains, spread over the
     // segments of a long sequence, were measured faster loading their own
@@ -1936,18 +1938,18 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const KdaChunk
         int track_len = -1;
         int64_t head_off = 0;
         auto item_ctx = [&]() {
-            slot = a.state_indices[n];
+            slot = a.slot_index(n);
             if (slot < 0 || static_cast<int64_t>(slot) >= a.num_slots) {
                 slot = 0;
             }
             track_slot = 0;
             track_len = -1;
             if (a.track_indices != nullptr) {
-                track_slot = a.track_indices[n];
+                track_slot = a.track_index(n);
                 if (track_slot <= 0 || static_cast<int64_t>(track_slot) >= a.num_slots) {
                     track_slot = 0;
                 } else {
-                    track_len = a.track_lens[n];
+                    track_len = a.track_length(n);
                 }
             }
             head_off = static_cast<int64_t>(h) * a.state_stride_head;
@@ -2880,7 +2882,7 @@ constexpr int kAffThreads = 256;
 // consecutive entries of a column of S_s ([v'][k], the pool's layout). Every
 // wave holds all of S_s as B operands; wave w forms rows [32w, 32w + 32) of
 // S_{s+1}, and the new columns pass to the next step through LDS.
-__global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const KdaChunkArgs a, char *ws,
+__global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const ChunkLaunch a, char *ws,
                                                                          int P, int W) {
     __shared__ float sb[2][16][DK + 4];  // S_{s+1} by step parity: [column][k], rows padded
     const int H = a.num_heads;
@@ -2895,18 +2897,18 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
     if (nch <= W) {
         return;  // segment 0 held the whole sequence and finished it
     }
-    int slot = a.state_indices[0];
+    int slot = a.slot_index(0);
     if (slot < 0 || static_cast<int64_t>(slot) >= a.num_slots) {
         slot = 0;
     }
     int track_slot = 0;
     int track_len = -1;
     if (a.track_indices != nullptr) {
-        track_slot = a.track_indices[0];
+        track_slot = a.track_index(0);
         if (track_slot <= 0 || static_cast<int64_t>(track_slot) >= a.num_slots) {
             track_slot = 0;
         } else {
-            track_len = a.track_lens[0];
+            track_len = a.track_length(0);
         }
     }
     const Layout LY = layout(a.num_tokens, 1, H);
@@ -3034,7 +3036,7 @@ constexpr int kAffCorrectChunks = 4;
 // hi + lo B fragments (64 KiB), each 16-row tile of O is split likewise, and
 // the product takes three passes (hi hi, hi lo, lo hi: about 2^-16 relative
 // per term). Wave w takes token rows [16w, 16w + 16) of each chunk.
-__global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const KdaChunkArgs a, char *ws, int P,
+__global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const ChunkLaunch a, char *ws, int P,
                                                                          int W) {
     __shared__ u32x4 sb[4][8][2][64];  // S_s B fragments: [K slice][column tile][hi, lo][lane]
     const int H = a.num_heads;
@@ -3396,8 +3398,8 @@ int check_args(const KdaChunkArgs *args) {
 // `pipeline` (ring = 2 win) K1 of segment s+1 runs on the library's side
 // stream while segment s is scanned, otherwise (ring >= win) the segments run
 // one after another on `st`.
-int launch(const KdaChunkArgs &a, char *ws, hipStream_t st, int ring, int win, bool pipeline, int first_seg = 0) {
-    KdaChunkArgs kargs = a;
+int launch(const ChunkLaunch &a, char *ws, hipStream_t st, int ring, int win, bool pipeline, int first_seg = 0) {
+    ChunkLaunch kargs = a;
     const int nrec = max_chunks(a.num_tokens, a.num_seqs);
     const int64_t pairs = static_cast<int64_t>(a.num_seqs) * a.num_heads;
     const int nt = scan_tiles(pairs, st);
@@ -3514,8 +3516,8 @@ int launch(const KdaChunkArgs &a, char *ws, hipStream_t st, int ring, int win, b
 // first pass (segment 0 from the pool, the later segments from zero and from
 // the identity), the serial combine, the parallel correction of the later
 // segments' outputs.
-int launch_affine(const KdaChunkArgs &a, char *ws, hipStream_t st, int P, int W) {
-    KdaChunkArgs kargs = a;
+int launch_affine(const ChunkLaunch &a, char *ws, hipStream_t st, int P, int W) {
+    ChunkLaunch kargs = a;
     const int H = a.num_heads;
     const int nrec = max_chunks(a.num_tokens, 1);
     const int nch_max = chunk_bound(a.num_tokens);
@@ -3598,12 +3600,17 @@ char *scratch_address(hipStream_t st) {
 
 extern "C" int kda_chunk_launch(const KdaChunkArgs *args, void *workspace, size_t workspace_bytes,
                                 void *stream) {
+    return kda_chunk_launch_wide(args, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int kda_chunk_launch_wide(const KdaChunkArgs *args, int32_t wide, void *workspace,
+                                     size_t workspace_bytes, void *stream) {
     using namespace kda::chunk;
     const int rc = check_args(args);
     if (rc != KDA_OK || args->num_seqs == 0) {
         return rc;
     }
-    const KdaChunkArgs &a = *args;
+    const ChunkLaunch a{*args, wide};
     if (workspace == nullptr || !aligned(workspace, 256)) {
         return KDA_ERR_WORKSPACE;
     }
@@ -3641,7 +3648,7 @@ extern "C" int kda_chunk_launch_noalloc(const KdaChunkArgs *args, void *stream) 
     if (rc != KDA_OK || args->num_seqs == 0) {
         return rc;
     }
-    const KdaChunkArgs &a = *args;
+    const ChunkLaunch a{*args, 0};
     const int T = a.num_tokens;
     const int H = a.num_heads;
     const bool whole = layout(T, a.num_seqs, H).total <= KDA_NOALLOC_SCRATCH_BYTES;

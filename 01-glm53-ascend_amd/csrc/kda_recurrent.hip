@@ -42,6 +42,8 @@ namespace {
 
 constexpr int kThreads = 256;
 
+using RecurrentLaunch = Launch<KdaRecurrentArgs>;
+
 // e^x as one v_exp_f32 of x*log2(e). The product's rounding puts the
 // relative error near |x| * 2^-24 plus the instruction's own ~1 ulp; a
 // result below the fp32 normal range may flush to zero.
@@ -203,7 +205,7 @@ __device__ __forceinline__ void store_row(T *p, const float (&x)[NP], int kc) {
 }
 
 template <int D, int L, int NP, typename TQK, typename TV, int GATE>
-__global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentArgs a) {
+__global__ __launch_bounds__(kThreads) void recurrent_kernel(const RecurrentLaunch a) {
     constexpr int E = D / L;           // K elements per lane
     constexpr int EV = E / 4;          // 16-byte vectors per lane and row
     constexpr int RPW = 64 / L;        // row groups per wave
@@ -236,11 +238,11 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
     const int row0 = vt * RB + rgw;  // rows row0 + RS*p, p < NP
     const int T = a.num_tokens;
 
-    int bos = a.cu_seqlens[n];
-    int eos = a.cu_seqlens[n + 1];
+    int bos = a.cu(n);
+    int eos = a.cu(n + 1);
     bos = bos < 0 ? 0 : (bos > T ? T : bos);
     eos = eos < bos ? bos : (eos > T ? T : eos);
-    int slot = a.state_indices[n];
+    int slot = a.slot_index(n);
     if (slot < 0 || static_cast<int64_t>(slot) >= a.num_slots) {
         slot = 0;
     }
@@ -284,11 +286,11 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
     int track_slot = 0;
     int track_len = -1;
     if (a.track_indices != nullptr) {
-        track_slot = a.track_indices[n];
+        track_slot = a.track_index(n);
         if (track_slot <= 0 || static_cast<int64_t>(track_slot) >= a.num_slots) {
             track_slot = 0;
         } else {
-            track_len = a.track_lens[n];
+            track_len = a.track_length(n);
         }
     }
     // State tiles are touched once per launch: streamed with nontemporal
@@ -625,7 +627,7 @@ __global__ __launch_bounds__(kThreads) void recurrent_kernel(const KdaRecurrentA
 // ---------------------------------------------------------------------------
 
 template <int D, int NP, int SW, typename TQK, typename TV, int GATE>
-__global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const KdaRecurrentArgs a) {
+__global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const RecurrentLaunch a) {
     constexpr int L = 16;
     constexpr int EV = D / L / 4;  // 16-byte vectors per lane and row
     constexpr int RB = 16 * NP;    // rows per workgroup
@@ -680,11 +682,11 @@ __global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const KdaRecu
     };
     const int T = a.num_tokens;
 
-    int bos = a.cu_seqlens[n];
-    int eos = a.cu_seqlens[n + 1];
+    int bos = a.cu(n);
+    int eos = a.cu(n + 1);
     bos = bos < 0 ? 0 : (bos > T ? T : bos);
     eos = eos < bos ? bos : (eos > T ? T : eos);
-    int slot = a.state_indices[n];
+    int slot = a.slot_index(n);
     if (slot < 0 || static_cast<int64_t>(slot) >= a.num_slots) {
         slot = 0;
     }
@@ -775,11 +777,11 @@ __global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const KdaRecu
     int track_slot = 0;
     int track_len = -1;
     if (a.track_indices != nullptr) {
-        track_slot = a.track_indices[n];
+        track_slot = a.track_index(n);
         if (track_slot <= 0 || static_cast<int64_t>(track_slot) >= a.num_slots) {
             track_slot = 0;
         } else {
-            track_len = a.track_lens[n];
+            track_len = a.track_length(n);
         }
     }
     auto store_state = [&](float *dst, bool vlayout) {
@@ -1023,7 +1025,7 @@ __global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const KdaRecu
 
 }
 
-using KernelFn = void (*)(const KdaRecurrentArgs);
+using KernelFn = void (*)(const RecurrentLaunch);
 
 // Tile shapes: (lanes per row L, rows per lane NP).
 enum Shape { kDecode16, kDecode8, kBlock16, kBlock64, kBlock128, kWave128, kD64Small, kD64Large };
@@ -1087,6 +1089,10 @@ bool aligned8(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0
 }  // namespace kda
 
 extern "C" int kda_recurrent_launch(const KdaRecurrentArgs *args, void *stream) {
+    return kda_recurrent_launch_wide(args, 0, stream);
+}
+
+extern "C" int kda_recurrent_launch_wide(const KdaRecurrentArgs *args, int32_t wide, void *stream) {
     using namespace kda;
     if (args == nullptr) {
         return KDA_ERR_INVALID_ARGUMENT;
@@ -1135,7 +1141,7 @@ extern "C" int kda_recurrent_launch(const KdaRecurrentArgs *args, void *stream) 
         return KDA_ERR_INVALID_ARGUMENT;
     }
 
-    KdaRecurrentArgs kargs = a;
+    RecurrentLaunch kargs{a, wide};
     if (kargs.head_begin < 0 || kargs.head_begin >= kargs.num_heads || kargs.head_count < 0) {
         return KDA_ERR_INVALID_ARGUMENT;
     }

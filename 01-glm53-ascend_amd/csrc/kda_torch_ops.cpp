@@ -18,9 +18,9 @@
 //
 // Each op validates what the kernels index against, in the reference's
 // order and with its message text (callers match substrings, e.g.
-// tests/integration/kda_ascendc_dispatch.py:52-58), narrows int64 metadata
-// to int32 on the device, allocates the output, and enqueues one launch on the
-// current stream. No host synchronization: unlike the reference chunk op
+// tests/integration/kda_ascendc_dispatch.py:52-58), allocates the output, and
+// enqueues one launch on the current stream (the kernels read int32 and int64
+// metadata alike). No host synchronization: unlike the reference chunk op
 // (kda_varlen_chunk.cpp:130-143), ragged lengths are accepted, so cu_seqlens
 // never has to be read back.
 
@@ -52,15 +52,41 @@ void *stream_of(const at::Tensor &t) {
     return static_cast<void *>(c10::hip::getCurrentHIPStream(t.device().index()).stream());
 }
 
-at::Tensor as_int32(const at::Tensor &t) {
-    return t.scalar_type() == at::kInt ? t.contiguous() : t.to(at::kInt).contiguous();
-}
+// A launch's metadata (int32 or int64, checked before), made contiguous where it
+// is not, and which of its arrays are int64 (KDA_WIDE_*): the kernels read
+// either, so no conversion is launched.
+struct Metadata {
+    int32_t wide = 0;  // first: the tensors' initialization sets its bits
+    at::Tensor indices, cu_seqlens;
+    std::optional<at::Tensor> track_indices, track_lens;
 
-std::optional<at::Tensor> as_int32_opt(const std::optional<at::Tensor> &t) {
-    return t.has_value() ? std::optional<at::Tensor>(as_int32(*t)) : std::nullopt;
-}
+    Metadata(const at::Tensor &idx, const at::Tensor &cu, const std::optional<at::Tensor> &track_idx,
+             const std::optional<at::Tensor> &lens)
+        : indices(take(idx, KDA_WIDE_STATE_INDICES)), cu_seqlens(take(cu, KDA_WIDE_CU_SEQLENS)) {
+        if (track_idx.has_value()) {
+            track_indices = take(*track_idx, KDA_WIDE_TRACK_INDICES);
+        }
+        if (lens.has_value()) {
+            track_lens = take(*lens, KDA_WIDE_TRACK_LENS);
+        }
+    }
 
-const int32_t *i32_ptr(const at::Tensor &t) { return t.data_ptr<int32_t>(); }
+    template <class Args> void set(Args &args) const {
+        args.state_indices = ptr(indices);
+        args.cu_seqlens = ptr(cu_seqlens);
+        if (track_indices.has_value()) {
+            args.track_indices = ptr(*track_indices);
+            args.track_lens = ptr(*track_lens);
+        }
+    }
+
+  private:
+    at::Tensor take(const at::Tensor &t, int32_t bit) {
+        wide |= t.scalar_type() == at::kLong ? bit : 0;
+        return t.contiguous();
+    }
+    static const int32_t *ptr(const at::Tensor &t) { return static_cast<const int32_t *>(t.data_ptr()); }
+};
 
 // One packed token batch [1, T, H, D] (the sglang contract; a leading batch
 // above one would otherwise be ignored), with T and the request count in the
@@ -148,8 +174,6 @@ struct PoolRef {
 PoolRef pool_ref(at::Tensor &pool) {
     return PoolRef{pool.data_ptr<float>(), pool.stride(0), pool.stride(1), pool.size(0)};
 }
-
-at::Tensor run_chunk(const char *op, KdaChunkArgs &args, const at::Tensor &q);
 
 // A prefill of K = V = 128 whose requests average at least this many tokens
 // runs in the chunked form (measured: 1024 tokens on 4 heads take ~1 ms
@@ -240,10 +264,7 @@ at::Tensor varlen_recurrent_impl(const char *op, const at::Tensor &A_log, const 
 
     check_on_gpu("q", q);
     const c10::DeviceGuard device_guard(q.device());  // launch on q's device
-    const at::Tensor idx32 = as_int32(indices);
-    const at::Tensor cu32 = as_int32(cu_seqlens);
-    const auto ti32 = as_int32_opt(track_indices);
-    const auto tl32 = as_int32_opt(track_lens);
+    const Metadata meta(indices, cu_seqlens, track_indices, track_lens);
     // Every token is written by the kernel (uncovered ones as zero), so the
     // output needs no fill: the reference's zeros_like is kept as a contract,
     // not as a memset.
@@ -290,13 +311,8 @@ at::Tensor varlen_recurrent_impl(const char *op, const at::Tensor &A_log, const 
         cargs.state_stride_slot = pr.stride_slot;
         cargs.state_stride_head = pr.stride_head;
         cargs.num_slots = pr.num_slots;
-        cargs.state_indices = i32_ptr(idx32);
-        cargs.cu_seqlens = i32_ptr(cu32);
+        meta.set(cargs);
         cargs.out = out.data_ptr();
-        if (ti32.has_value()) {
-            cargs.track_indices = i32_ptr(*ti32);
-            cargs.track_lens = i32_ptr(*tl32);
-        }
         cargs.scale = static_cast<float>(scale);
         cargs.lower_bound = static_cast<float>(lower_bound);
         cargs.num_seqs = static_cast<int32_t>(N);
@@ -307,7 +323,7 @@ at::Tensor varlen_recurrent_impl(const char *op, const at::Tensor &A_log, const 
         cargs.v_dtype = KDA_BF16;
         cargs.gate_mode = KDA_GATE_RAW;
         cargs.qk_l2norm = 1;
-        check_ok(kda_chunk_launch(&cargs, route_buf->data_ptr(), route_ws, stream_of(q)), op);
+        check_ok(kda_chunk_launch_wide(&cargs, meta.wide, route_buf->data_ptr(), route_ws, stream_of(q)), op);
         return out;
     }
 
@@ -323,8 +339,7 @@ at::Tensor varlen_recurrent_impl(const char *op, const at::Tensor &A_log, const 
     args.state_stride_slot = pr.stride_slot;
     args.state_stride_head = pr.stride_head;
     args.num_slots = pr.num_slots;
-    args.state_indices = i32_ptr(idx32);
-    args.cu_seqlens = i32_ptr(cu32);
+    meta.set(args);
     args.out = out.data_ptr();
     if (save_mid) {
         at::Tensor mid = *intermediate;
@@ -334,10 +349,6 @@ at::Tensor varlen_recurrent_impl(const char *op, const at::Tensor &A_log, const 
         args.mid_stride_head = mid.stride(2);
         args.mid_rows = mid.size(0);
         args.mid_steps = mid.size(1);
-    }
-    if (ti32.has_value()) {
-        args.track_indices = i32_ptr(*ti32);
-        args.track_lens = i32_ptr(*tl32);
     }
     args.scale = static_cast<float>(scale);
     args.lower_bound = static_cast<float>(lower_bound);
@@ -351,7 +362,7 @@ at::Tensor varlen_recurrent_impl(const char *op, const at::Tensor &A_log, const 
     args.v_dtype = KDA_BF16;
     args.gate_mode = KDA_GATE_RAW;
     args.qk_l2norm = 1;
-    check_ok(kda_recurrent_launch(&args, stream_of(q)), op);
+    check_ok(kda_recurrent_launch_wide(&args, meta.wide, stream_of(q)), op);
     return out;
 }
 
@@ -391,12 +402,12 @@ at::Tensor kda_varlen_recurrent_v2(const at::Tensor &A_log, const at::Tensor &a,
 // kda_varlen_chunk
 // ---------------------------------------------------------------------------
 
-at::Tensor run_chunk(const char *op, KdaChunkArgs &args, const at::Tensor &q) {
+at::Tensor run_chunk(const char *op, KdaChunkArgs &args, int32_t wide, const at::Tensor &q) {
     const size_t ws = kda_chunk_workspace_bytes(args.num_tokens, args.num_seqs, args.num_heads,
                                                 args.head_dim);
     at::Tensor workspace =
         at::empty({static_cast<int64_t>(ws > 0 ? ws : 1)}, q.options().dtype(at::kByte));
-    check_ok(kda_chunk_launch(&args, workspace.data_ptr(), ws, stream_of(q)), op);
+    check_ok(kda_chunk_launch_wide(&args, wide, workspace.data_ptr(), ws, stream_of(q)), op);
     return workspace;
 }
 
@@ -435,10 +446,7 @@ at::Tensor varlen_chunk_impl(const char *op, const at::Tensor &A_log, const at::
     const int64_t N = indices.numel();
     check_on_gpu("q", q);
     const c10::DeviceGuard device_guard(q.device());  // launch on q's device
-    const at::Tensor idx32 = as_int32(indices);
-    const at::Tensor cu32 = as_int32(cu_seqlens);
-    const auto ti32 = as_int32_opt(track_indices);
-    const auto tl32 = as_int32_opt(track_lens);
+    const Metadata meta(indices, cu_seqlens, track_indices, track_lens);
     at::Tensor out = at::empty_like(v);
     // No request: every token is uncovered, so zero. No tokens but some
     // requests still launch: a prefix tracked at length 0 receives the
@@ -459,13 +467,8 @@ at::Tensor varlen_chunk_impl(const char *op, const at::Tensor &A_log, const at::
     args.state_stride_slot = pr.stride_slot;
     args.state_stride_head = pr.stride_head;
     args.num_slots = pr.num_slots;
-    args.state_indices = i32_ptr(idx32);
-    args.cu_seqlens = i32_ptr(cu32);
+    meta.set(args);
     args.out = out.data_ptr();
-    if (ti32.has_value()) {
-        args.track_indices = i32_ptr(*ti32);
-        args.track_lens = i32_ptr(*tl32);
-    }
     args.scale = static_cast<float>(scale);
     args.lower_bound = static_cast<float>(lower_bound);
     args.num_seqs = static_cast<int32_t>(N);
@@ -476,7 +479,7 @@ at::Tensor varlen_chunk_impl(const char *op, const at::Tensor &A_log, const at::
     args.v_dtype = KDA_BF16;
     args.gate_mode = KDA_GATE_RAW;
     args.qk_l2norm = 1;
-    run_chunk(op, args, q);
+    run_chunk(op, args, meta.wide, q);
     return out;
 }
 
@@ -585,10 +588,7 @@ at::Tensor kda_prepared_varlen_recurrent(const at::Tensor &q, const at::Tensor &
     }
     check_on_gpu("q", q);
     const c10::DeviceGuard device_guard(q.device());  // launch on q's device
-    const at::Tensor idx32 = as_int32(initial_state_indices);
-    const at::Tensor cu32 = as_int32(cu_seqlens);
-    const auto ti32 = as_int32_opt(track_state_indices);
-    const auto tl32 = as_int32_opt(track_state_lens);
+    const Metadata meta(initial_state_indices, cu_seqlens, track_state_indices, track_state_lens);
     at::Tensor out = at::empty_like(v);
     // No request: every token is uncovered, so zero. No tokens but some
     // requests still launch: a prefix tracked at length 0 receives the
@@ -607,8 +607,7 @@ at::Tensor kda_prepared_varlen_recurrent(const at::Tensor &q, const at::Tensor &
     args.state_stride_slot = pr.stride_slot;
     args.state_stride_head = pr.stride_head;
     args.num_slots = pr.num_slots;
-    args.state_indices = i32_ptr(idx32);
-    args.cu_seqlens = i32_ptr(cu32);
+    meta.set(args);
     args.out = out.data_ptr();
     if (intermediate_state.has_value()) {
         at::Tensor mid = *intermediate_state;
@@ -618,10 +617,6 @@ at::Tensor kda_prepared_varlen_recurrent(const at::Tensor &q, const at::Tensor &
         args.mid_stride_head = mid.stride(2);
         args.mid_rows = mid.size(0);
         args.mid_steps = mid.size(1);
-    }
-    if (ti32.has_value()) {
-        args.track_indices = i32_ptr(*ti32);
-        args.track_lens = i32_ptr(*tl32);
     }
     args.scale = static_cast<float>(scale);
     args.num_seqs = static_cast<int32_t>(N);
@@ -634,7 +629,7 @@ at::Tensor kda_prepared_varlen_recurrent(const at::Tensor &q, const at::Tensor &
     args.v_dtype = p.qk_dtype;
     args.gate_mode = KDA_GATE_LOG;
     args.qk_l2norm = use_qk_l2norm ? 1 : 0;
-    check_ok(kda_recurrent_launch(&args, stream_of(q)), op);
+    check_ok(kda_recurrent_launch_wide(&args, meta.wide, stream_of(q)), op);
     return out;
 }
 
@@ -654,10 +649,7 @@ at::Tensor kda_prepared_varlen_chunk(const at::Tensor &q, const at::Tensor &k,
     const int64_t N = initial_state_indices.numel();
     check_on_gpu("q", q);
     const c10::DeviceGuard device_guard(q.device());  // launch on q's device
-    const at::Tensor idx32 = as_int32(initial_state_indices);
-    const at::Tensor cu32 = as_int32(cu_seqlens);
-    const auto ti32 = as_int32_opt(track_state_indices);
-    const auto tl32 = as_int32_opt(track_state_lens);
+    const Metadata meta(initial_state_indices, cu_seqlens, track_state_indices, track_state_lens);
     at::Tensor out = at::empty_like(v);
     // No request: every token is uncovered, so zero. No tokens but some
     // requests still launch: a prefix tracked at length 0 receives the
@@ -676,13 +668,8 @@ at::Tensor kda_prepared_varlen_chunk(const at::Tensor &q, const at::Tensor &k,
     args.state_stride_slot = pr.stride_slot;
     args.state_stride_head = pr.stride_head;
     args.num_slots = pr.num_slots;
-    args.state_indices = i32_ptr(idx32);
-    args.cu_seqlens = i32_ptr(cu32);
+    meta.set(args);
     args.out = out.data_ptr();
-    if (ti32.has_value()) {
-        args.track_indices = i32_ptr(*ti32);
-        args.track_lens = i32_ptr(*tl32);
-    }
     args.scale = static_cast<float>(scale);
     args.num_seqs = static_cast<int32_t>(N);
     args.num_tokens = static_cast<int32_t>(p.T);
@@ -692,7 +679,7 @@ at::Tensor kda_prepared_varlen_chunk(const at::Tensor &q, const at::Tensor &k,
     args.v_dtype = KDA_BF16;
     args.gate_mode = KDA_GATE_LOG;
     args.qk_l2norm = use_qk_l2norm ? 1 : 0;
-    run_chunk(op, args, q);
+    run_chunk(op, args, meta.wide, q);
     return out;
 }
 
@@ -785,13 +772,8 @@ void prepared_recurrent(const at::Tensor &qn, const at::Tensor &kn, const at::Te
                 "(stride(3)==1, stride(2)==D), got strides (", state.stride(2), ", ", state.stride(3),
                 ")");
     const PoolRef pr = pool_ref(state);
-    const at::Tensor idx32 = as_int32(indices);
-    const at::Tensor cu32 = as_int32(starts);
-    std::optional<at::Tensor> ti32, tl32;
-    if (track_state) {
-        ti32 = as_int32(*track_indices);
-        tl32 = as_int32(*track_lens);
-    }
+    const std::optional<at::Tensor> none;
+    const Metadata meta(indices, starts, track_state ? track_indices : none, track_state ? track_lens : none);
     KdaRecurrentArgs args{};
     args.q = qn.data_ptr();
     args.k = kn.data_ptr();
@@ -802,13 +784,8 @@ void prepared_recurrent(const at::Tensor &qn, const at::Tensor &kn, const at::Te
     args.state_stride_slot = pr.stride_slot;
     args.state_stride_head = pr.stride_head;
     args.num_slots = pr.num_slots;
-    args.state_indices = i32_ptr(idx32);
-    args.cu_seqlens = i32_ptr(cu32);
+    meta.set(args);
     args.out = out.data_ptr();
-    if (ti32.has_value()) {
-        args.track_indices = i32_ptr(*ti32);
-        args.track_lens = i32_ptr(*tl32);
-    }
     args.scale = 1.0f;  // qn arrives with the scale folded in
     args.num_seqs = static_cast<int32_t>(N);
     args.num_tokens = static_cast<int32_t>(T);
@@ -821,7 +798,7 @@ void prepared_recurrent(const at::Tensor &qn, const at::Tensor &kn, const at::Te
     args.gate_mode = KDA_GATE_DECAY;
     args.qk_l2norm = 0;
     args.state_v_contiguous = k_contig ? 0 : 1;
-    check_ok(kda_recurrent_launch(&args, stream_of(qn)), op);
+    check_ok(kda_recurrent_launch_wide(&args, meta.wide, stream_of(qn)), op);
 }
 
 }  // namespace

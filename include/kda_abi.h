@@ -32,6 +32,7 @@
  *   cu_seqlens      int32 [N+1], non-decreasing, cu_seqlens[N] <= T;
  *   indices         int32 [N]; entries outside [0, num_slots) are treated as
  *                   slot 0 (the kernels never address outside the pool).
+ *                   The *_wide entry points also take int64 metadata.
  *
  * With num_tokens == 0 the token pointers (q, k, v, gate, beta, out) may be
  * null: the requests still run, so a prefix tracked at length 0 receives the
@@ -144,6 +145,18 @@ typedef struct KdaRecurrentArgs {
  * anywhere: aligned ones move as vectors, others element by element. */
 int kda_recurrent_launch(const KdaRecurrentArgs *args, void *stream);
 
+/* Metadata arrays of a launch that hold int64 entries (their pointers cast to
+ * const int32_t *). The kernels read the entries' low 32 bits, as a conversion
+ * to int32 would keep them. */
+#define KDA_WIDE_CU_SEQLENS 1
+#define KDA_WIDE_STATE_INDICES 2
+#define KDA_WIDE_TRACK_INDICES 4
+#define KDA_WIDE_TRACK_LENS 8
+
+/* kda_recurrent_launch with int64 metadata arrays: `wide` is a sum of KDA_WIDE_*
+ * (0: all int32). No counterpart in the reference, which converts them first. */
+int kda_recurrent_launch_wide(const KdaRecurrentArgs *args, int32_t wide, void *stream);
+
 typedef struct KdaChunkArgs {
     const void *q;        /* [T,H,D], qk_dtype */
     const void *k;        /* [T,H,D], qk_dtype */
@@ -221,6 +234,10 @@ size_t kda_chunk_workspace_bytes(int32_t num_tokens, int32_t num_seqs,
  * multiples of 4 elements; q, k, v and out 8 bytes; gate 8 (RAW) or 16. */
 int kda_chunk_launch(const KdaChunkArgs *args, void *workspace,
                      size_t workspace_bytes, void *stream);
+
+/* kda_chunk_launch with int64 metadata arrays (see kda_recurrent_launch_wide). */
+int kda_chunk_launch_wide(const KdaChunkArgs *args, int32_t wide, void *workspace,
+                          size_t workspace_bytes, void *stream);
 
 /* Bytes of the static device scratch behind kda_chunk_launch_noalloc. */
 #define KDA_NOALLOC_SCRATCH_BYTES (64u * 1024u * 1024u)
