@@ -45,8 +45,8 @@
 // (hi hi, hi lo, lo hi): Akk and Aqk; T^T kd and Aqk T take T, kd and Aqk
 // as fp16 hi + lo pairs (~2^-22) in three passes.
 // The record the scan reads holds every matrix operand as fp16 (11-bit
-// significands) with a power-of-two scale per fragment or row tile: e^G k,
-// q e^G, (T^T kd)^T and Aqk T. The scan meets them with S_j as fp16 (scaled
+// significands) with a power-of-two scale: one for all of e^G k, one for
+// q e^G, one per row tile for (T^T kd)^T and Aqk T. The scan meets them with S_j as fp16 (scaled
 // per 32-row slice; S itself stays fp32) for (e^G k) S and (q e^G) S, and
 // with y as fp16 hi + lo (~2^-22) for (T^T kd)^T y and (Aqk T) y.
 //
@@ -227,8 +227,8 @@ __device__ __forceinline__ void split_bf16x8(const float x[8], bf16x8 &hi, bf16x
     lo = as_bf16x8(l);
 }
 
-// fp16 fragments carry x * 2^sh, with sh chosen per fragment (or per S
-// slice) from its largest magnitude m so that m * 2^sh lies in [2^13, 2^14):
+// fp16 fragments carry x * 2^sh, with sh chosen per row tile, S slice or
+// operand from its largest magnitude (or a bound) m so that m * 2^sh lies in [2^13, 2^14):
 // well inside fp16's range, full 11-bit significands down to 2^-27 m.
 __device__ __forceinline__ int f16_shift(float m) {
     if (!(m > 0.f)) {
@@ -1627,7 +1627,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 //                     j+1's parity between B1(j) and B2(j) (every reader of
 //                     that stage's previous chunk j-1 finished before B1(j)),
 //                     then issue the loads of chunk j+3. The recurrence never
-//                     waits to issue a global load.
+//                     waits to issue a global load. The loaders arrive last at
+//                     both barriers (8192 tokens, 32 heads: 115-130 clocks of
+//                     wait against the chain's 390 and 200), so what bounds a
+//                     step is the 57 KiB that pass the CU's vector-memory path
+//                     and the LDS stage, not the chain.
 // The affine form's first pass runs a lean variant: the chain waves load
 // their e^G k and (T^T kd)^T fragments, and the output waves their Aqk T,
 // from the record themselves a chunk ahead (every fragment has one reader
