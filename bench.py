@@ -429,7 +429,7 @@ def run_raw_decode(steps, warmup, min_settle, check):
         roofline=dict(bound="hbm", achieved=gbs, peak=HBM_PEAK_GBS, unit="GB/s",
                       frac=gbs / HBM_PEAK_GBS, traffic=traffic, traffic_source=traffic_src,
                       algorithmic_bytes_per_launch=RAW_DEC_BYTES,
-                      kernel="recurrent_kernel<128,32,2,strided rows,decode,bf16,bf16,RAW>"))
+                      kernel="recurrent_kernel<128,32,2,bf16,bf16,RAW>"))
 
 
 # ---------------------------------------------------------------------------
@@ -935,7 +935,7 @@ def main():
         roofline=dict(
             bound="hbm", achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s",
             frac=achieved / HBM_PEAK_GBS, traffic=traffic, traffic_source=traffic_src,
-            kernel="recurrent_kernel<128,32,2,strided rows,decode,bf16,bf16,LOG>",
+            kernel="recurrent_kernel<128,32,2,bf16,bf16,LOG>",
             algorithmic_bytes_per_launch=DEC_BYTES,
             event_us_per_call=dec["event_us_per_call"],
             source_sha256=dec_sha,
