@@ -3033,22 +3033,30 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
 }
 
 // Chunks per correction workgroup (they share the staged S_s).
-constexpr int kAffCorrectChunks = 4;
+constexpr int kAffCorrectThreads = 512;
 
-// One workgroup per (later segment s, head, kAffCorrectChunks of the
-// segment's chunks): o_t = bf16(o'_t + O_t S_s). S_s is staged once as bf16
+// One workgroup per (later segment s, head, `per` of the segment's chunks): o_t = bf16(o'_t + O_t S_s). S_s is staged once as bf16
 // hi + lo B fragments (64 KiB), each 16-row tile of O is split likewise, and
 // the product takes three passes (hi hi, hi lo, lo hi: about 2^-16 relative
-// per term). Wave w takes token rows [16w, 16w + 16) of each chunk.
-__global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const ChunkLaunch a, char *ws, int P,
-                                                                         int W) {
+// per term). Wave w takes token rows [16 (w % 4), + 16) of chunks w / 4,
+// w / 4 + 2, ...
+//
+// The two output planes bound it (63 MB at 16384 tokens on 4 heads, 10 us),
+// with few workgroups to keep them coming (192 there). So eight waves share a
+// staged S_s, two chunks in flight, and column r of tile nt stands for value
+// 8 r + nt: a lane's results of a row are then eight neighbours, o' arrives
+// as two vectors and o leaves as two instead of eight elements each. Four
+// waves, four chunks and single elements took 22 us there, this 13.5 (a raw
+// prefill of 16384 tokens, graph replays: 4 heads 135.7 -> 127.2 us).
+__global__ __launch_bounds__(kAffCorrectThreads) void chunk_affine_correct_kernel(const ChunkLaunch a, char *ws, int P,
+                                                                               int W, int per) {
     __shared__ u32x4 sb[4][8][2][64];  // S_s B fragments: [K slice][column tile][hi, lo][lane]
     const int H = a.num_heads;
-    const int groups = (W + kAffCorrectChunks - 1) / kAffCorrectChunks;
+    const int groups = (W + per - 1) / per;
     const int s = 1 + static_cast<int>(blockIdx.x) / (groups * H);
     const int rest = static_cast<int>(blockIdx.x) % (groups * H);
     const int h = rest % H;
-    const int c_lo = s * W + (rest / H) * kAffCorrectChunks;
+    const int c_lo = s * W + (rest / H) * per;
     int bos, eos;
     seq_bounds(a, 0, bos, eos);
     const int nch = (eos - bos + BT - 1) / BT;
@@ -3056,7 +3064,7 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const
     if (s >= P || c_lo >= seg_hi) {
         return;
     }
-    const int c_hi = c_lo + kAffCorrectChunks < seg_hi ? c_lo + kAffCorrectChunks : seg_hi;
+    const int c_hi = c_lo + per < seg_hi ? c_lo + per : seg_hi;
     const AffLayout AL = aff_layout(a.num_tokens, H, P);
     const float *S = reinterpret_cast<const float *>(ws + AL.start + static_cast<size_t>(H) * DK * DK * 4 * (s - 1)) +
                      static_cast<size_t>(h) * DK * DK;
@@ -3065,16 +3073,16 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const
     uint16_t *out = static_cast<uint16_t *>(a.out);
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int w = tid >> 6;
+    const int w = (tid >> 6) & 3;
     const int r = lane & 15;
     const int gq = lane >> 4;
     // S_s as B fragments: lane (r, gq) of fragment (slice sl, tile nt) holds
-    // S[k = 32 sl + kperm(gq, e)][v = 16 nt + r]; S is [V][K], so each half
+    // S[k = 32 sl + kperm(gq, e)][v = 8 r + nt]; S is [V][K], so each half
     // of the eight is one float4 run of K
-    for (int f = w; f < 32; f += 4) {
+    for (int f = tid >> 6; f < 32; f += 8) {
         const int sl = f & 3;
         const int nt = f >> 2;
-        const float *col = S + static_cast<int64_t>(16 * nt + r) * DK + 32 * sl + 4 * gq;
+        const float *col = S + static_cast<int64_t>(8 * r + nt) * DK + 32 * sl + 4 * gq;
         const float4 x0 = *reinterpret_cast<const float4 *>(col);
         const float4 x1 = *reinterpret_cast<const float4 *>(col + 16);
         const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
@@ -3084,7 +3092,7 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const
         sb[sl][nt][1][lane] = as_u32x4(lo);
     }
     __syncthreads();
-    for (int c = c_lo; c < c_hi; ++c) {
+    for (int c = c_lo + (tid >> 8); c < c_hi; c += 2) {
         const int t0 = bos + BT * c;
         const int len = eos - t0 < BT ? eos - t0 : BT;
         // A: row 16 w + r of O (rows past the chunk's end read its last row;
@@ -3099,14 +3107,13 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const
         }
         // o' of this lane's outputs, loaded before the products need them
         // (rows past the chunk's end read its last row)
-        float oz[8][4];
+        float4 oz[4][2];
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = 16 * w + 4 * gq + i < len ? 16 * w + 4 * gq + i : len - 1;
-                oz[nt][i] = Oz[(static_cast<int64_t>(t0 + t) * H + h) * DK + 16 * nt + r];
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int t = 16 * w + 4 * gq + i < len ? 16 * w + 4 * gq + i : len - 1;
+            const float *zrow = Oz + (static_cast<int64_t>(t0 + t) * H + h) * DK + 8 * r;
+            oz[i][0] = *reinterpret_cast<const float4 *>(zrow);
+            oz[i][1] = *reinterpret_cast<const float4 *>(zrow + 4);
         }
         bf16x8 ah[4], al[4];
 #pragma unroll
@@ -3115,23 +3122,31 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_correct_kernel(const
                                 ox[sl][1].x, ox[sl][1].y, ox[sl][1].z, ox[sl][1].w};
             split_bf16x8(x, ah[sl], al[sl]);
         }
-#pragma unroll 2
+        f32x4 acc[8];
+#pragma unroll
         for (int nt = 0; nt < 8; ++nt) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+            acc[nt] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int sl = 0; sl < 4; ++sl) {
                 const bf16x8 bh = as_bf16x8(sb[sl][nt][0][lane]);
                 const bf16x8 bl = as_bf16x8(sb[sl][nt][1][lane]);
-                acc = mfma(ah[sl], bh, acc);
-                acc = mfma(ah[sl], bl, acc);
-                acc = mfma(al[sl], bh, acc);
+                acc[nt] = mfma(ah[sl], bh, acc[nt]);
+                acc[nt] = mfma(ah[sl], bl, acc[nt]);
+                acc[nt] = mfma(al[sl], bh, acc[nt]);
             }
-            // lane (r, gq) holds C[4 gq + i][r]: token 16 w + 4 gq + i, column 16 nt + r
+        }
+        // lane (r, gq) holds C[4 gq + i][r] of tile nt: token 16 w + 4 gq + i, column 8 r + nt
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = 16 * w + 4 * gq + i;
-                if (t < len) {
-                    out[(static_cast<int64_t>(t0 + t) * H + h) * DK + 16 * nt + r] = f32_to_bf16(oz[nt][i] + acc[i]);
+        for (int i = 0; i < 4; ++i) {
+            const int t = 16 * w + 4 * gq + i;
+            if (t < len) {
+                uint16_t *row = out + (static_cast<int64_t>(t0 + t) * H + h) * DK + 8 * r;
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    const float4 z = oz[i][half];
+                    *reinterpret_cast<uint2 *>(row + 4 * half) =
+                        make_uint2(pack_bf16x2(z.x + acc[4 * half][i], z.y + acc[4 * half + 1][i]),
+                                   pack_bf16x2(z.z + acc[4 * half + 2][i], z.w + acc[4 * half + 3][i]));
                 }
             }
         }
@@ -3551,10 +3566,19 @@ int launch_affine(const ChunkLaunch &a, char *ws, hipStream_t st, int P, int W) 
                         dim3(kAffThreads), cparams, 0, st) != hipSuccess) {
         return KDA_ERR_LAUNCH;
     }
-    const int64_t later = static_cast<int64_t>(P - 1) * ((W + kAffCorrectChunks - 1) / kAffCorrectChunks) * H;
+    // Two chunks per workgroup of the correction, one per four waves, while two
+    // workgroups per CU (their S_s takes 64 KiB of LDS) hold them all; then
+    // four, which stage S_s half as often (graph replays, 16384 tokens: 1 head
+    // 83.4 us against 87.2 with four, 4 heads 127.2 against 128.5, 8 heads
+    // 246.0 against 247.0; 32768 on 4 heads 270.7 against 268.9; eight chunks
+    // 93.6, 133.2, 249.0 and 269.9).
+    auto groups = [&](int per) { return static_cast<int64_t>(P - 1) * ((W + per - 1) / per) * H; };
+    int per = groups(2) <= 2 * static_cast<int64_t>(device_cus(st)) ? 2 : 4;
+    const int64_t later = groups(per);
+    void *oparams[] = {&kargs, &ws, &sp, &sw, &per};
     if (nch_max > W && later > 0 &&
         hipLaunchKernel(reinterpret_cast<const void *>(chunk_affine_correct_kernel), dim3(static_cast<unsigned>(later)),
-                        dim3(kAffThreads), cparams, 0, st) != hipSuccess) {
+                        dim3(kAffCorrectThreads), oparams, 0, st) != hipSuccess) {
         return KDA_ERR_LAUNCH;
     }
     return KDA_OK;
