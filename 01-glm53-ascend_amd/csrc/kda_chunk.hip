@@ -2880,10 +2880,13 @@ constexpr int kAffThreads = 256;
 // tracked scan states combined the same way), and the final state into the
 // pool. The products run on the fp32 MFMA (v_mfma_f32_16x16x4f32, lane (r, g)
 // supplying A[r][g] and B[g][r] of each 4-wide K step, C as for the bf16
-// tiles) with the K index v' permuted: at step kk lane (r, g) supplies v' =
-// 32 g + kk, so its A values are 32 consecutive entries of a row of Phi
-// (stored [k][v'] by the identity-start scan) and its B values 32
-// consecutive entries of a column of S_s ([v'][k], the pool's layout). Every
+// tiles) with the K index v' permuted: at step 4 i + e lane (r, g) supplies v' =
+// 16 i + 4 g + e, so its A values are vectors of a row of Phi (stored [k][v']
+// by the identity-start scan), its B values vectors of a column of S_s
+// ([v'][k], the pool's layout), and the four lanes of a row read 64
+// neighbouring bytes: each wave's loads of Phi bound a step as much as its
+// products (three steps on 4 heads 13.4 us with 32 consecutive entries per
+// lane, each 16-byte piece in a line of its own; 12.1 so). Every
 // wave holds all of S_s as B operands; wave w forms rows [32w, 32w + 32) of
 // S_{s+1}, and the new columns pass to the next step through LDS.
 __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const ChunkLaunch a, char *ws,
@@ -2926,15 +2929,15 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
     const int r = lane & 15;
     const int gq = lane >> 4;
     const int col = 16 * g + r;  // this lane's column of S (B and C operands)
-    // S_s as B operands: bv[i][e] = S_s[32 gq + 4 i + e][col]; S_1 from the
+    // S_s as B operands: bv[i][e] = S_s[16 i + 4 gq + e][col]; S_1 from the
     // carry area ([V][K])
     float4 bv[8];
     const float *carry = reinterpret_cast<const float *>(ws + LY.carry) + hoff;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        bv[i] = load4(carry + static_cast<int64_t>(col) * DK + 32 * gq + 4 * i);
+        bv[i] = load4(carry + static_cast<int64_t>(col) * DK + 16 * i + 4 * gq);
     }
-    // A operands of this wave's two row tiles t: Phi[16 (2w + t) + r][32 gq + 4 i + e];
+    // A operands of this wave's two row tiles t: Phi[16 (2w + t) + r][16 i + 4 gq + e];
     // C initial values: Z[16 (2w + t) + 4 gq + e][col]
     struct Ops {
         float4 A[2][8];
@@ -2945,7 +2948,7 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
         for (int t = 0; t < 2; ++t) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                op.A[t][i] = load4(M + static_cast<int64_t>(16 * (2 * w + t) + r) * DK + 32 * gq + 4 * i);
+                op.A[t][i] = load4(M + static_cast<int64_t>(16 * (2 * w + t) + r) * DK + 16 * i + 4 * gq);
             }
         }
 #pragma unroll
@@ -2971,13 +2974,13 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
         }
     };
     const int64_t head_off = static_cast<int64_t>(h) * a.state_stride_head;
-    // this wave's quarter of a state held as B operands (rows 32 gq + 4 i,
+    // this wave's quarter of a state held as B operands (rows 16 i + 4 gq,
     // i = 2 (w & 3) .. +1), into [V][K] at `dst`
     auto store_b = [&](float *dst) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             if ((i >> 1) == w) {
-                *reinterpret_cast<float4 *>(dst + static_cast<int64_t>(col) * DK + 32 * gq + 4 * i) = bv[i];
+                *reinterpret_cast<float4 *>(dst + static_cast<int64_t>(col) * DK + 16 * i + 4 * gq) = bv[i];
             }
         }
     };
@@ -3015,7 +3018,7 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            bv[i] = *reinterpret_cast<const float4 *>(&buf[r][32 * gq + 4 * i]);
+            bv[i] = *reinterpret_cast<const float4 *>(&buf[r][16 * i + 4 * gq]);
         }
     };
     Ops oa, ob;
