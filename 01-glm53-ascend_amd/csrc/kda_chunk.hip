@@ -45,8 +45,8 @@
 // (hi hi, hi lo, lo hi): Akk and Aqk; T^T kd and Aqk T take T, kd and Aqk
 // as fp16 hi + lo pairs (~2^-22) in three passes.
 // The record the scan reads holds every matrix operand as fp16 (11-bit
-// significands) with a power-of-two scale: one for all of e^G k, one for
-// q e^G, one per row tile for (T^T kd)^T and Aqk T. The scan meets them with S_j as fp16 (scaled
+// significands) with a power-of-two scale per fragment group or row tile: e^G k,
+// q e^G, (T^T kd)^T and Aqk T. The scan meets them with S_j as fp16 (scaled
 // per 32-row slice; S itself stays fp32) for (e^G k) S and (q e^G) S, and
 // with y as fp16 hi + lo (~2^-22) for (T^T kd)^T y and (Aqk T) y.
 //
@@ -103,11 +103,11 @@ constexpr int kOffSc = kOffGl + DK * 4;           // fp32 scale block [128], ind
 constexpr int kRecBytes = kOffSc + 512;           // 56320
 // Scale block: 2^-shift of each fp16 fragment group, and the bound the scan
 // derives y's scale from (|y| <= max|v| + kel1 max|S|).
-constexpr int kScKe = 0;     // [1] e^G k, all fragments
-constexpr int kScQg = 1;     // [1] q e^G, all fragments
-constexpr int kScKel1 = 2;   // [1] a bound of max_t sum_k |(e^G k)[t][k]|
+constexpr int kScKe = 0;     // [8] e^G k row tile mt, channel half h (slices 2h, 2h + 1): 2 mt + h
+constexpr int kScQg = 8;     // [8] q e^G, likewise
 constexpr int kScKd = 32;    // [8] (T^T kd)^T row tile mk (both token slices)
 constexpr int kScAq = 40;    // [4] Aqk T row tile mt (both token slices)
+constexpr int kScKel1 = 44;  // [1] a bound of max_t sum_k |(e^G k)[t][k]|
 // Largest of four nonnegative values (magnitudes), compared as their bit
 // patterns: no quieting of the operands as fmaxf needs for values it did not
 // produce itself.
@@ -227,8 +227,8 @@ __device__ __forceinline__ void split_bf16x8(const float x[8], bf16x8 &hi, bf16x
     lo = as_bf16x8(l);
 }
 
-// fp16 fragments carry x * 2^sh, with sh chosen per row tile, S slice or
-// operand from its largest magnitude (or a bound) m so that m * 2^sh lies in [2^13, 2^14):
+// fp16 fragments carry x * 2^sh, with sh chosen per fragment group, row tile or
+// S slice from its largest magnitude m so that m * 2^sh lies in [2^13, 2^14):
 // well inside fp16's range, full 11-bit significands down to 2^-27 m.
 __device__ __forceinline__ int f16_shift(float m) {
     if (!(m > 0.f)) {
@@ -238,6 +238,14 @@ __device__ __forceinline__ int f16_shift(float m) {
     (void)frexpf(m, &e);  // m = f 2^e, f in [0.5, 1)
     const int sh = 14 - e;
     return sh < -120 ? -120 : (sh > 120 ? 120 : sh);
+}
+// The same of a magnitude given as its bits, wave-uniform: scalar instructions
+// (no search for zero, where any shift serves; a group holding an infinity
+// keeps its finite values' scale near 1).
+__device__ __forceinline__ int f16_shift_bits(uint32_t m) {
+    const int e = m >= 0x7f800000u ? 126 : static_cast<int>(m >> 23);
+    const int sh = 140 - e;
+    return sh > 120 ? 120 : sh;
 }
 __device__ __forceinline__ f16x8 to_f16x8(const float x[8], int sh) {
     f16x8 h;
@@ -299,6 +307,58 @@ __device__ __forceinline__ float wave_max_mag(float x) {
     const uint32_t b = max(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), 32)),
                            static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), 48)));
     return __uint_as_float(max(a, b));
+}
+
+// Within each 16-lane row, the row's largest value in every lane.
+__device__ __forceinline__ uint32_t row_max(uint32_t u) {
+    u = max(u, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(u), kDppQuadXor1, 0xf, 0xf, true)));
+    u = max(u, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(u), kDppQuadXor2, 0xf, 0xf, true)));
+    u = max(u, static_cast<uint32_t>(
+                   __builtin_amdgcn_mov_dpp(static_cast<int>(u), kDppRowHalfMirror, 0xf, 0xf, true)));
+    return max(u, static_cast<uint32_t>(
+                      __builtin_amdgcn_mov_dpp(static_cast<int>(u), kDppRowMirror, 0xf, 0xf, true)));
+}
+__device__ __forceinline__ uint32_t lane_of(uint32_t u, int l) {
+    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u), l));
+}
+
+// The shifts of two fragment groups from each lane's largest magnitudes x and y:
+// after one swap of half waves the lower half reduces x and the upper half y.
+__device__ __forceinline__ void wave_shifts(float x, float y, int &sx, int &sy) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    const uint32_t u = row_max(max(static_cast<uint32_t>(p[0]), static_cast<uint32_t>(p[1])));
+    sx = f16_shift_bits(max(lane_of(u, 0), lane_of(u, 16)));
+    sy = f16_shift_bits(max(lane_of(u, 32), lane_of(u, 48)));
+}
+
+// The same of four groups: a swap of half waves, one of rows, and each row of
+// 16 lanes reduces one group.
+__device__ __forceinline__ void wave_shifts(float x, float y, float z, float w, int &sx, int &sy, int &sz, int &sw) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(z), __float_as_uint(w), false, false);
+    // rows 0, 1: x, rows 2, 3: y; and z, w
+    const auto t = __builtin_amdgcn_permlane16_swap(max(static_cast<uint32_t>(p[0]), static_cast<uint32_t>(p[1])),
+                                                    max(static_cast<uint32_t>(q[0]), static_cast<uint32_t>(q[1])), false,
+                                                    false);
+    // rows x, z, y, w
+    const uint32_t u = row_max(max(static_cast<uint32_t>(t[0]), static_cast<uint32_t>(t[1])));
+    sx = f16_shift_bits(lane_of(u, 0));
+    sz = f16_shift_bits(lane_of(u, 16));
+    sy = f16_shift_bits(lane_of(u, 32));
+    sw = f16_shift_bits(lane_of(u, 48));
+}
+
+template <int N>
+__device__ __forceinline__ float max_mag(const float (&x)[N][8]) {
+    float m = 0.f;
+#pragma unroll
+    for (int f = 0; f < N; ++f) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            m = fmaxf(m, fabsf(x[f][e]));
+        }
+    }
+    return m;
 }
 
 // Per 16-bit half, the larger of m and the magnitude of a bf16 value (as bits).
@@ -652,12 +712,9 @@ struct PrepShared {
     float beta[BT];
     float gsum[4][DK];  // each wave's two row groups' decay sums (the cumsum's carries)
     alignas(16) int far[4];     // per wave: some anchor factor of its rows spans > kExactExp2
-    // per wave: largest magnitude of its k and q rows as given (bf16 bits; not
-    // used when they are normalized), largest positive log2 decay of a token
-    // (0 for decays, which are <= 0)
-    alignas(16) uint32_t kmax[4];
-    alignas(16) uint32_t qmax[4];
-    alignas(16) float grow[4];
+    // [channel half][row tile]: max over the tile's rows of the sum of |e^G k|
+    // over the half's channels
+    alignas(16) float kel1[2][4];
 };
 static_assert(sizeof(PrepShared) <= 80 * 1024, "two prepare workgroups per CU");
 
@@ -850,29 +907,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             *reinterpret_cast<float4 *>(&sm.u.early.K[t][4 * kc]) =
                 make_float4(k4.x * rn, k4.y * rn, k4.z * rn, k4.w * rn);
         }
-        // The extremes the record's fp16 scales are bounded by: max |k|, and how
-        // far a token's decay goes above 1 (never, when g <= 0)
-        if (!norm) {
-            uint32_t m = 0;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                m = max_mag_bf16x2(max_mag_bf16x2(m, kraw[i].x), kraw[i].y);
-            }
-            sm.kmax[wave] = __float_as_uint(wave_max_mag(__uint_as_float(max(m & 0xffffu, m >> 16))));
-        }
-        {
-            int m = 0;  // positive floats order as their bits, negative ones are below 0
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                m = max(max(max(m, __float_as_int(g4[i].x)), __float_as_int(g4[i].y)),
-                        max(__float_as_int(g4[i].z), __float_as_int(g4[i].w)));
-            }
-            float up = 0.f;
-            if (__builtin_expect(__ballot(m > 0) != 0ull, 0)) {
-                up = wave_max_mag(__int_as_float(m)) * kLog2e;
-            }
-            sm.grow[wave] = up;
-        }
         // S2, the in-chunk cumsum of the log2 decay: this lane's eight rows in
         // registers, then the row groups before it: its half-wave partner
         // (rg - 1, for odd rg) by a lane exchange, earlier waves' pairs
@@ -953,52 +987,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 sm.u.early.qss[sh][16 * (ii == 0 ? IA : 3 - IA) + r] = ss;
             }
         }
-    } else {
-        uint32_t m = 0;
-#pragma unroll
-        for (int ii = 0; ii < 2; ++ii) {
-#pragma unroll
-            for (int q2 = 0; q2 < 2; ++q2) {
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    m = max_mag_bf16x2(max_mag_bf16x2(m, qraw[ii][q2][e].x), qraw[ii][q2][e].y);
-                }
-            }
-        }
-        sm.qmax[wave] = __float_as_uint(wave_max_mag(__uint_as_float(max(m & 0xffffu, m >> 16))));
     }
     lds_barrier();
-
-    // Power-of-two scales of the record's fp16 operands from bounds rather than
-    // from their own largest values, whose search cost K1 a reduction over the
-    // wave per fragment group (six of them, and 60 maxima per lane): |e^G k| and
-    // |kd| <= max|k|, |q e^G| <= max|q|, |Aqk| <= 128 max|k| max|q| (all times
-    // 2^up where a decay goes above 1); normalized rows have norm 1. fp16
-    // keeps its 11 bits down to 2^-28 of the bound, so a bound some powers of
-    // two above the largest value loses nothing.
-    // (With the residuals of bf16_residual and without the clamps of the anchor
-    // factors, which the exact form makes needless: 417 of 4502 VALU
-    // instructions less; 8192 tokens on 32 heads 285.8 -> 273.8 us in all.)
-    int ksh, qsh, aqsh;
-    float kel1;
-    {
-        auto max4_bf16 = [](const uint32_t *p) {
-            const uint4 u = *reinterpret_cast<const uint4 *>(p);
-            return __uint_as_float(max(max(u.x, u.y), max(u.z, u.w)) << 16);
-        };
-        const float km = norm ? 1.f : max4_bf16(sm.kmax);
-        const float qm = (norm ? 1.f : max4_bf16(sm.qmax)) * fabsf(a.scale);
-        const int up = static_cast<int>(
-            fminf(ceilf(static_cast<float>(BT) * max4_mag(*reinterpret_cast<const float4 *>(sm.grow))), 100.f));
-        const int sk = f16_shift(km);
-        const int sq = f16_shift(qm);
-        ksh = __builtin_amdgcn_readfirstlane(sk - up);
-        qsh = __builtin_amdgcn_readfirstlane(sq - up);
-        // max|k| < 2^(14 - sk), max|q| < 2^(14 - sq): 128 of their products stay
-        // below 2^14 under 2^(sk + sq - 21); normalized rows' below max|q|
-        aqsh = __builtin_amdgcn_readfirstlane((norm ? sq : max(min(sk + sq - 21, 120), -120)) - up);
-        kel1 = ldexpf(128.f * km, up);
-    }
 
     // 8 channels {32s + kperm(gq, e)} of one row: two 16-byte reads each
     // from the (normalized) k and the cumsum tiles.
@@ -1075,6 +1065,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // stay in registers until the k and cumsum tiles are dead (after S4), and
     // the halves are then summed in LT.
     f32x4 pk[2][4], pq[2][4];  // this half's partials of pair (I, J): Akk, Aqk
+    float *sc = reinterpret_cast<float *>(rec + kOffSc);
+    bf16x8 Rh[2][2], Rl[2][2], Qh[2][2], Ql[2][2];
+    float anc[2][2][8];
+    float qg[2][2][8];  // q e^G of this half's two slices
+    float ke[2][2][8];  // e^G k of the same rows and channels
+    float l1[2];  // this lane's share of its row's sum of |e^G k| over the half
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii) {
         const int I = ii == 0 ? IA : 3 - IA;
@@ -1095,14 +1091,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         // 8 consecutive tokens decay by less than 2^kMaxExp2 (about 87 nat).
         // Beyond that the products may not be finite; the exact form replaces
         // every one of them.
-        float anc[2][8];
 #pragma unroll
         for (int sl = 0; sl < 2; ++sl) {
-            load_g8(16 * I + kAnchorRow, 2 * sh + sl, anc[sl]);
+            load_g8(16 * I + kAnchorRow, 2 * sh + sl, anc[ii][sl]);
         }
-        bf16x8 Rh[2], Rl[2], Qh[2], Ql[2];
-        float qg[2][8];  // q e^G of this half's two slices
-        float ke[2][8];  // e^G k of the same rows and channels
 #pragma unroll
         for (int sl = 0; sl < 2; ++sl) {
             const int s = 2 * sh + sl;
@@ -1111,21 +1103,48 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             load_g8(ri, s, gg);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float ex = ex2(gg[e] - anc[sl][e]);
+                const float ex = ex2(gg[e] - anc[ii][sl][e]);
                 const float eg = ex2(gg[e]);
                 const float qn = qv[sl][e] * qscale;
                 rv[e] = kk[e] * ex;
                 qa[e] = qn * ex;
-                qg[sl][e] = qn * eg;
-                ke[sl][e] = kk[e] * eg;
+                qg[ii][sl][e] = qn * eg;
+                ke[ii][sl][e] = kk[e] * eg;
             }
-            split_bf16x8(rv, Rh[sl], Rl[sl]);
-            split_bf16x8(qa, Qh[sl], Ql[sl]);
+            split_bf16x8(rv, Rh[ii][sl], Rl[ii][sl]);
+            split_bf16x8(qa, Qh[ii][sl], Ql[ii][sl]);
         }
-        store_frags_f16<2>(rec, kOffQg, I * 4 + 2 * sh, qsh, lane, qg);
+    }
+    // Each tile and half has scales of its own, from its largest values: a bound
+    // over the chunk (max |k|, max |q|, the largest step of a growing decay) is cheaper, but a
+    // row far below it, or after one growing token every row, loses its bits.
+    // Both blocks' four groups share one reduction (K1 of 8192 tokens, 32
+    // heads: 121 us, with a reduction for each group 126, with bounds 123).
+    int qsh[2], ksh[2];
+    wave_shifts(max_mag(qg[0]), max_mag(ke[0]), max_mag(qg[1]), max_mag(ke[1]), qsh[0], ksh[0], qsh[1], ksh[1]);
+#pragma unroll
+    for (int ii = 0; ii < 2; ++ii) {
+        const int I = ii == 0 ? IA : 3 - IA;
         // e^G k: the A fragments of row tile I, slices 2sh and 2sh+1, for the
-        // scan's (e^G k) S
-        store_frags_f16<2>(rec, kOffKe, I * 4 + 2 * sh, ksh, lane, ke);
+        // scan's (e^G k) S; q e^G alike. One scale each for this tile and half.
+        store_frags_f16<2>(rec, kOffQg, I * 4 + 2 * sh, qsh[ii], lane, qg[ii]);
+        store_frags_f16<2>(rec, kOffKe, I * 4 + 2 * sh, ksh[ii], lane, ke[ii]);
+        if (lane == 0) {
+            sc[kScQg + 2 * I + sh] = ldexpf(1.f, -qsh[ii]);
+            sc[kScKe + 2 * I + sh] = ldexpf(1.f, -ksh[ii]);
+        }
+        l1[ii] = 0.f;
+#pragma unroll
+        for (int sl = 0; sl < 2; ++sl) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                l1[ii] += fabsf(ke[ii][sl][e]);
+            }
+        }
+    }
+#pragma unroll
+    for (int ii = 0; ii < 2; ++ii) {
+        const int I = ii == 0 ? IA : 3 - IA;
         // pairs (I, J), J <= I, over this half's channels
 #pragma unroll
         for (int J = 0; J < (ii == 0 ? 4 : 2); ++J) {
@@ -1143,7 +1162,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 load_g8(rj, s, gg);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    cv[e] = kk[e] * ex2(anc[sl][e] - gg[e]);
+                    cv[e] = kk[e] * ex2(anc[ii][sl][e] - gg[e]);
                 }
                 bf16x8 Ch, Cl;
                 split_bf16x8(cv, Ch, Cl);
@@ -1151,16 +1170,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 // (2^-9 per term) reaches T, and where the decay is weak the
                 // state keeps every chunk's error (8.5e-4 against 3.5e-4 of
                 // the final state's max after 16384 tokens at g ~ -1e-4)
-                akk = mfma(Rh[sl], Ch, akk);  // Akk[16I + 4gq + e][16J + r]
-                akk = mfma(Rh[sl], Cl, akk);
-                akk = mfma(Rl[sl], Ch, akk);
-                aqt = mfma(Ch, Qh[sl], aqt);  // Aqk[16I + r][16J + 4gq + e]
-                aqt = mfma(Ch, Ql[sl], aqt);
-                aqt = mfma(Cl, Qh[sl], aqt);
+                akk = mfma(Rh[ii][sl], Ch, akk);  // Akk[16I + 4gq + e][16J + r]
+                akk = mfma(Rh[ii][sl], Cl, akk);
+                akk = mfma(Rl[ii][sl], Ch, akk);
+                aqt = mfma(Ch, Qh[ii][sl], aqt);  // Aqk[16I + r][16J + 4gq + e]
+                aqt = mfma(Ch, Ql[ii][sl], aqt);
+                aqt = mfma(Cl, Qh[ii][sl], aqt);
             }
             // lane (r, gq) holds Akk[16I + 4gq + e][16J + r] and Aqk[16I + r][16J + 4gq + e]
             pk[ii][J] = akk;
             pq[ii][J] = aqt;
+        }
+    }
+    {
+        // the rows' sums over the four lane groups (lower half wave: block IA's,
+        // upper: 3 - IA's) and their largest
+        const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(l1[0]), __float_as_uint(l1[1]), false, false);
+        const float x = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        const uint32_t u = row_max(__float_as_uint(__uint_as_float(q[0]) + __uint_as_float(q[1])));
+        if ((lane & 31) == 0) {
+            sm.kel1[sh][lane == 0 ? IA : 3 - IA] = __uint_as_float(u);
         }
     }
     // ---- S4: kd fragments (kept for S6), e^(G_last), tracking operands, e^G k
@@ -1174,9 +1204,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     };
     // kd[t][16mk + r] = k_t e^(G_last - G_t) for the rows t = 32s + kperm(gq, e)
-    // (B fragments of T^T kd, mk = 2 wave + tt), fp16 hi + lo scaled by 2^ksh;
-    // S6 uses them from registers.
+    // (B fragments of T^T kd, mk = 2 wave + tt), fp16 hi + lo with one
+    // power-of-two scale 2^-shift per mk; S6 uses them from registers.
     u32x4 kdh[2][2], kdl[2][2];
+    int kdsh[2];
     auto to_frags = [&](const float (&x)[2][8], u32x4 (&fh)[2], u32x4 (&fl)[2], int shift) {
 #pragma unroll
         for (int s = 0; s < 2; ++s) {
@@ -1186,23 +1217,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             fl[s] = as_u32x4(lo);
         }
     };
+    {
+        float x[2][2][8];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-        const int mk = 2 * wave + tt;
-        const int k = 16 * mk + r;
-        const float gl = sm.u.early.G[BT - 1][k];
-        float x[2][8];
+        for (int tt = 0; tt < 2; ++tt) {
+            const int mk = 2 * wave + tt;
+            const int k = 16 * mk + r;
+            const float gl = sm.u.early.G[BT - 1][k];
 #pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            float kr[8];
-            kd_rows(s, mk, kr);
+            for (int s = 0; s < 2; ++s) {
+                float kr[8];
+                kd_rows(s, mk, kr);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int t = 32 * s + kperm(gq, e);
-                x[s][e] = kr[e] * ex2(gl - sm.u.early.G[t][k]);
+                for (int e = 0; e < 8; ++e) {
+                    const int t = 32 * s + kperm(gq, e);
+                    x[tt][s][e] = kr[e] * ex2(gl - sm.u.early.G[t][k]);
+                }
             }
         }
-        to_frags(x, kdh[tt], kdl[tt], ksh);
+        wave_shifts(max_mag(x[0]), max_mag(x[1]), kdsh[0], kdsh[1]);
+        to_frags(x[0], kdh[0], kdl[0], kdsh[0]);
+        to_frags(x[1], kdh[1], kdl[1], kdsh[1]);
     }
     if (tid < DK) {
         reinterpret_cast<float *>(rec + kOffGl)[tid] = ex2(sm.u.early.G[BT - 1][tid]);
@@ -1214,6 +1249,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     bool tracked = false;
     char *tr = nullptr;
     u32x4 kth[2][2], ktl[2][2];
+    int ktsh[2] = {0, 0};
     if (a.track_indices != nullptr) {
         const int ts = a.track_index(n);
         const int tl = a.track_length(n);
@@ -1237,7 +1273,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                         x[s][e] = t < rr ? kr[e] * ex2(gr - sm.u.early.G[t][k]) : 0.f;
                     }
                 }
-                to_frags(x, kth[tt], ktl[tt], ksh);
+                ktsh[tt] = f16_shift_bits(__float_as_uint(wave_max_mag(max_mag(x))));
+                to_frags(x, kth[tt], ktl[tt], ktsh[tt]);
             }
             if (tid < DK) {
                 reinterpret_cast<float *>(tr + kTrOffGl)[tid] = ex2(sm.u.early.G[rr - 1][tid]);
@@ -1390,6 +1427,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             sm.u.mid.X[16 * gq + i][16 * gq + r] = acc[i];
         }
     } else {
+        if (tid == 64) {
+            const float4 h0 = *reinterpret_cast<const float4 *>(sm.kel1[0]);
+            const float4 h1 = *reinterpret_cast<const float4 *>(sm.kel1[1]);
+            sc[kScKel1] = max4_mag(h0.x + h1.x, h0.y + h1.y, h0.z + h1.z, h0.w + h1.w);
+        }
         // X's six upper 16x16 blocks (I, J > I) are zero, one float4 per store
         for (int f = tid - 64; f < 6 * 64; f += kThreads - 64) {
             const int blk = f >> 6;  // (0,1) (0,2) (0,3) (1,2) (1,3) (2,3)
@@ -1404,6 +1446,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // = Aqk[16 wave + r][32s + kperm(g, e)] (zero above the diagonal). Here, since
     // three of the four waves wait for the diagonal blocks.
     u32x4 aqh[2], aql[2];
+    int aqsh;
     {
         const int row = 16 * wave + r;
         float ax[2][8];
@@ -1417,6 +1460,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                 ax[s][e] = 32 * s + kperm(gq, e) <= row ? xv[e] : 0.f;
             }
         }
+        aqsh = f16_shift_bits(__float_as_uint(wave_max_mag(max_mag(ax))));
         to_frags(ax, aqh, aql, aqsh);
     }
     lds_barrier();
@@ -1489,12 +1533,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // output (Aqk T) y. Both are stored as A fragments: a pair of 16x16
     // result tiles over token rows [32s, 32s+16) and [32s+16, 32s+32) is the
     // A fragment of token slice s.
-    float *sc = reinterpret_cast<float *>(rec + kOffSc);
-    if (tid == 0) {
-        sc[kScKe] = ldexpf(1.f, -ksh);
-        sc[kScQg] = ldexpf(1.f, -qsh);
-        sc[kScKel1] = kel1;
-    }
     {
         // T^T fragments of row tile tt = wave (both token slices): lane (r, g)
         // element e holds T[32s + kperm(g, e)][16 wave + r] (zero where the
@@ -1563,7 +1601,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int mk = 2 * wave + tt;
         float x[2][8];
         int ex[4];
-        ttb(kdh[tt], kdl[tt], ksh, x, 3, ex);
+        ttb(kdh[tt], kdl[tt], kdsh[tt], x, 3, ex);
         store_frags_f16_exp<2>(rec, kOffKd, mk * 2, sc + kScKd + mk, lane, x, ex);
     }
     if (tracked) {
@@ -1572,7 +1610,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int mk = 2 * wave + tt;
             float x[2][8];
             int ex[4];
-            ttb(kth[tt], ktl[tt], ksh, x, 3, ex);
+            ttb(kth[tt], ktl[tt], ktsh[tt], x, 3, ex);
             store_frags_f16_exp<2>(tr, kTrOffKd, mk * 2, reinterpret_cast<float *>(tr + kTrOffSc) + mk, lane, x,
                                    ex);
         }
@@ -1731,6 +1769,29 @@ __device__ __forceinline__ f16x8 stage_frag(const char *st, int f, int lane) {
 // chain loads the next item's initial state a whole item ahead; what a
 // workgroup per item paid at its start (about 3.9 us: dispatch, the first
 // loads, the pipeline's fill and drain) is paid once per workgroup.
+//
+// A row tile's scales of e^G k or q e^G: two, one per channel half. At 16 columns
+// a lane loads one and both are broadcast when needed: a wave's loads
+// of the same eight bytes cost the vector-memory and LDS paths twice as much
+// as of four, and those bound a step there (8192 tokens, 32 heads: scan 140.9 us
+// against 142.5; 65,536 tokens, 16 heads: 1238 against 1254). At 32 columns, with more
+// work per step, the broadcasts cost more than they save (16 sequences, 32
+// heads: 360 us against 354).
+template <bool PICK> struct HalfScales;
+template <> struct HalfScales<true> {
+    float x;
+    __device__ __forceinline__ void load(const float *p, int lane) { x = p[lane & 1]; }
+    __device__ __forceinline__ float2 get() const {
+        return make_float2(__uint_as_float(lane_of(__float_as_uint(x), 0)),
+                           __uint_as_float(lane_of(__float_as_uint(x), 1)));
+    }
+};
+template <> struct HalfScales<false> {
+    float2 x;
+    __device__ __forceinline__ void load(const float *p, int) { x = *reinterpret_cast<const float2 *>(p); }
+    __device__ __forceinline__ float2 get() const { return x; }
+};
+
 template <int NT, bool SEG, bool AFF = false, bool PERS = false>
 __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLaunch a, const char *ws,
                                                                   int ring, int s_lo, int s_hi) {
@@ -2073,7 +2134,8 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLau
         struct OpsB {
             f16x8 Kef[4];
             f32x4 vv[NT];
-            float kesc, vmax, kel1;
+            HalfScales<NT == 1> kesc;
+            float vmax, kel1;
         };
         auto read_b = [&](OpsB &op, int p) {
             const char *st = sm.stg[p];
@@ -2101,7 +2163,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLau
             }
             const float4 um = *reinterpret_cast<const float4 *>(&sm.vmax[p][0]);
             op.vmax = max4_mag(um);
-            op.kesc = sc[kScKe];
+            op.kesc.load(sc + kScKe + 2 * wr, lane);
             op.kel1 = sc[kScKel1];
         };
         // chunk j (of the item, PERS) in the stage of parity p
@@ -2157,7 +2219,8 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLau
             const float4 ss = *reinterpret_cast<const float4 *>(&sm.sscale[p][0]);
             const int sv = f16_shift(ob.vmax + ob.kel1 * max4_mag(sx));
             const float inv_v = ldexpf(1.f, -sv);
-            const float fw[4] = {ob.kesc * ss.x, ob.kesc * ss.y, ob.kesc * ss.z, ob.kesc * ss.w};
+            const float2 kesc = ob.kesc.get();
+            const float fw[4] = {kesc.x * ss.x, kesc.x * ss.y, kesc.y * ss.z, kesc.y * ss.w};
             f16x8 Kd[2][2];
             f32x4 gl[2];
             float2 kdsc;
@@ -2462,7 +2525,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLau
         struct OpsO {
             f16x8 Qg[4];
             f16x8 Aq[2];
-            float qsc;
+            HalfScales<NT == 1> qsc;
         };
         Cur cl;  // PERS: load_out's position (one chunk ahead)
         Cur co;  // PERS: finish's position (one chunk behind)
@@ -2481,7 +2544,7 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLau
                 op.Aq[0] = as_f16x8(aq[aq_frag(wr, 0) * 64 + lane]);
                 op.Aq[1] = as_f16x8(aq[aq_frag(wr, wr >= 2 ? 1 : 0) * 64 + lane]);
             }
-            op.qsc = *reinterpret_cast<const float *>(rec + kOffSc + 4 * kScQg);
+            op.qsc.load(reinterpret_cast<const float *>(rec + kOffSc) + kScQg + 2 * wr, lane);
         };
         auto aqk_y = [&](const OpsO &op, int j) {
             const int p = j & 1;
@@ -2594,7 +2657,8 @@ __global__ __launch_bounds__(kScanThreads) void chunk_scan_kernel(const ChunkLau
             }
             f32x4 Pn[NT];
             const float4 ss = *reinterpret_cast<const float4 *>(&sm.sscale[p][0]);
-            const float fq[4] = {cur.qsc * ss.x, cur.qsc * ss.y, cur.qsc * ss.z, cur.qsc * ss.w};
+            const float2 qsc = cur.qsc.get();
+            const float fq[4] = {qsc.x * ss.x, qsc.x * ss.y, qsc.y * ss.z, qsc.y * ss.w};
 #pragma unroll
             for (int ct = 0; ct < NT; ++ct) {
                 f32x4 acc[4];
