@@ -784,19 +784,32 @@ __global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const Recurre
             track_len = a.track_length(n);
         }
     }
+    // The stores' addresses are formed where they are used: hoisted out of the token
+    // loop (three places store a state, in two layouts with decay gates) they cost 20
+    // to 40 registers, and with fp32 inputs a workgroup per CU: 64-row tiles took 138
+    // to 144, three per CU (512 x 3 tokens, decay gates: 17.3 us; now up to 120 and
+    // four: 14.2), 128-row ones 170 to 176, two. The others have room for them, and at
+    // many pairs fewer waves stream the states better (8192 x 2, 32-row tiles: 177
+    // us with four workgroups per CU, 184 with five).
+    constexpr bool kFormHere = GATE == KDA_GATE_DECAY || (sizeof(TQK) == 4 && NP >= 4);
     auto store_state = [&](float *dst, bool vlayout) {
+        int rs = row0;
+        int ks = 4 * kc;
+        if constexpr (kFormHere) {
+            asm volatile("" : "+v"(rs), "+v"(ks));
+        }
 #pragma unroll
         for (int p = 0; p < NP; ++p) {
 #pragma unroll
             for (int j = 0; j < EV; ++j) {
                 if (vlayout) {
-                    float *e = dst + static_cast<int64_t>(koff(j)) * D + row0 + p;
+                    float *e = dst + static_cast<int64_t>((ks + 4 * L * j)) * D + rs + p;
                     e[0] = S[p][j].x;
                     e[D] = S[p][j].y;
                     e[2 * D] = S[p][j].z;
                     e[3 * D] = S[p][j].w;
                 } else {
-                    store4_stream(dst + static_cast<int64_t>(row0 + p) * D + koff(j), S[p][j]);
+                    store4_stream(dst + static_cast<int64_t>(rs + p) * D + (ks + 4 * L * j), S[p][j]);
                 }
             }
         }

@@ -90,3 +90,33 @@ def test_prepared_blocks_with_checkpoints(gpu_ops, heads, n, steps, dtype):
     for i, length in enumerate(lengths):
         assert torch.equal(mid[i, length - 1], pool[int(case.indices[i])]), "the last checkpoint is the final state"
         assert (mid[i, length:] == 7.0).all(), "steps beyond the request stay"
+
+
+@pytest.mark.parametrize("k_contiguous", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,steps", [(32, 3), (64, 5), (75, 4), (100, 3), (160, 3), (300, 9), (512, 4)])
+def test_decay_blocks(gpu_ops, n, steps, dtype, k_contiguous):
+    """``prepared_recurrent`` (four heads) over its tiles, on both pool layouts,
+    with ragged lengths, a padding request, uncovered tokens and tracked prefixes."""
+    H, D = 4, 128
+    lengths = [steps - (i % 3 if i % 4 == 1 else 0) for i in range(n)]
+    case = C.prepared_case(H, lengths, dtype=torch.float32, slots=2 * n + 1, seed=19)
+    indices = case.indices.clone()
+    indices[2] = 0
+    track = _track(lengths)
+    track = [torch.tensor(x, dtype=torch.int32) for x in track]
+    pool = C.to_dev(case.pool, DEV) if k_contiguous else case.pool.contiguous().to(DEV)
+    T = case.q.shape[1]
+    pad = lambda x: torch.cat([x, x[:, :2]], 1).to(DEV)  # noqa: E731  two tokens no request covers
+    v = case.v.to(dtype)
+    out = torch.full((1, T + 2, H, D), 3.0, dtype=dtype, device=DEV)
+    gpu_ops.prepared_recurrent(pad(case.q * case.scale), pad(case.k), pad(v), pad(case.g.exp()), pad(case.beta), out, pool,
+                               indices.to(DEV), case.cu_seqlens.to(DEV), track[0].to(DEV), track[1].to(DEV), True, 0)
+    ref_pool = C.clone_pool(case.pool)
+    ref = R.kda_recurrent(case.q * case.scale, case.k, v.float(), case.g, case.beta, state_pool=ref_pool,
+                          state_indices=indices, cu_seqlens=case.cu_seqlens, out_dtype=torch.float32,
+                          track_state_indices=track[0], track_state_lens=track[1])
+    assert (out[:, T:] == 3.0).all(), "uncovered rows stay"
+    check = C.assert_out if dtype == torch.bfloat16 else C.assert_rel
+    check(out[:, :T].cpu(), ref, TOL, "output")
+    C.assert_rel(pool.cpu(), ref_pool, TOL, "states")
