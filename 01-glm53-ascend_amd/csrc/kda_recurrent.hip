@@ -636,7 +636,9 @@ __global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const Recurre
     constexpr int SR = BTOK * NP;  // rows of the sharing waves
     constexpr int VP = SR / L;     // v values a lane stages
     static_assert(D % RB == 0 && (SW == 1 || SW == 4) && VP >= 1, "whole row tiles");
-    // D = 64 keeps the correctly rounded expf of its one-token form.
+    // D = 64 keeps its one-token form's expf (about 1 ulp); at D = 128 the one-token
+    // form uses expf too, so there a token's state and output depend in their last bits
+    // on whether the batch holds more than one token per request.
     auto dexp = [](float x) { return D == 128 ? fexp(x) : expf(x); };
 
     // one block's prepared tokens: [token][channel], and [token][row of the
@@ -1040,8 +1042,10 @@ __global__ __launch_bounds__(kThreads) void recurrent_block_kernel(const Recurre
 
 using KernelFn = void (*)(const RecurrentLaunch);
 
-// Tile shapes: (lanes per row L, rows per lane NP).
-enum Shape { kDecode16, kDecode8, kBlock16, kBlock64, kBlock128, kWave128, kD64Small, kD64Large };
+// Tile shapes, by the rows a workgroup covers.
+enum Shape {
+    kDecode16, kDecode8, kBlock16, kBlock32, kBlock64, kBlock128, kWave64, kWave128, kD64Small, kD64Large
+};
 
 template <int D, typename TQK, typename TV, int GATE>
 KernelFn pick_shape(Shape shape) {
@@ -1050,11 +1054,19 @@ KernelFn pick_shape(Shape shape) {
             case kDecode16: return recurrent_kernel<D, 32, 2, TQK, TV, GATE>;
             case kDecode8: return recurrent_kernel<D, 32, 1, TQK, TV, GATE>;
             case kBlock16: return recurrent_block_kernel<D, 1, 4, TQK, TV, GATE>;
+            case kBlock32: return recurrent_block_kernel<D, 2, 4, TQK, TV, GATE>;
             case kBlock64: return recurrent_block_kernel<D, 4, 4, TQK, TV, GATE>;
             case kBlock128: return recurrent_block_kernel<D, 8, 4, TQK, TV, GATE>;
-            case kWave128: return recurrent_block_kernel<D, 8, 1, TQK, TV, GATE>;
-            default: return nullptr;
+            default: break;
         }
+        if constexpr (GATE == KDA_GATE_RAW) {  // prepared gates are not launched with these
+            switch (shape) {
+                case kWave64: return recurrent_block_kernel<D, 4, 1, TQK, TV, GATE>;
+                case kWave128: return recurrent_block_kernel<D, 8, 1, TQK, TV, GATE>;
+                default: break;
+            }
+        }
+        return nullptr;
     } else {
         switch (shape) {
             case kD64Large: return recurrent_kernel<D, 16, 4, TQK, TV, GATE>;
@@ -1093,6 +1105,111 @@ KernelFn pick_kernel(int gate, int qk_dtype, int v_dtype, Shape shape) {
         return nullptr;
     }
     return nullptr;
+}
+
+// The tile shape, by tokens per sequence (their mean) and (sequence, head) pairs.
+// Measured on MI355X as graph replays over pools that rotate through 1 GiB, in
+// microseconds, raw gates on bf16, log gates on bf16 and fp32 and decay gates at
+// 64 to 16384 pairs and 2 to 16 tokens (ragged: 20 to 120); "loop" is a token loop
+// without shared blocks, which the block shapes replaced.
+//
+// One token (decode), D = 128: 32-lane rows, 2 rows per lane: 16-row tiles, eight
+// workgroups per pair, which stream the state fastest (256 x 1, H=32: 173,
+// against 182 with 32-row tiles); 8-row tiles below 128 pairs.
+//
+// Several tokens, D = 128. What a tile shares is the token's preparation: long with
+// raw gates (four exponentials and a reciprocal per channel, the norms), short with
+// prepared ones. Below that, what counts is how many workgroups there are, whether
+// all are resident at once (256 CUs hold 256 pairs of 32-row tiles, 512 of 64-row
+// ones, 768 of 128-row ones), and how they stream the states.
+Shape tile_shape(const KdaRecurrentArgs &a, int64_t pairs) {
+    const int64_t seqs = a.num_seqs;
+    const int64_t ntok = a.num_tokens;
+    auto tokens = [&](int n) { return ntok <= n * seqs; };  // up to n a sequence
+    if (a.head_dim != 128) {
+        // 64-row tiles are one workgroup per pair, 16-row tiles four (2 x 37-63
+        // tokens, H=4: 17 against 25; 64 x 4, H=16: 14.9 against 9.1)
+        if (tokens(1)) {
+            return pairs >= 2048 ? kD64Large : kD64Small;
+        }
+        return pairs >= 256 ? kBlock64 : kBlock16;
+    }
+    if (tokens(1)) {
+        return pairs < 128 ? kDecode8 : kDecode16;
+    }
+    if (a.gate_mode == KDA_GATE_RAW) {
+        // few pairs: 16-row tiles spread a step over most CUs (32 x 4: 5.13, 32-row
+        // tiles 5.15, loop 6.1), from 48 pairs 32-row tiles fill them with half the
+        // preparations (48 x 2: 4.8 against 5.2; 256 x 2: 8.0 against 8.8 with
+        // 64-row tiles, loop 8.5; 256 x 20-120: 63 against 82, loop 170)
+        if (pairs <= 32) {
+            return kBlock16;
+        }
+        if (pairs <= 256) {
+            return kBlock32;
+        }
+        // 512 x 2: 13.9, 128-row tiles 14.5, loop 17.1; 512 x 16: 29.2, 30.9,
+        // loop 57; long sequences, bound by VALU issue, stay with their
+        // occupancy (2048 x 20-120: 401 against 418, loop 728)
+        if (pairs <= 512 || !tokens(16)) {
+            return kBlock64;
+        }
+        // 128-row tiles prepare a token once per pair (640 x 2: 16.1 against 19.8
+        // with 64-row tiles, loop 19.3; 1536 x 4: 42.2, 45.1, 46.3; 4096 x 6:
+        // 108.6, 109.0, 131). From 2048 pairs the state's traffic bounds up to
+        // four tokens, and a barrier only couples the waves' loads (one wave
+        // sharing, 4096 x 2: 95.9 against 104, loop 96.6; 4096 x 4: 99.4, 105.5,
+        // 107). At two tokens the third round of 128-row tiles is short just
+        // below that (1856 x 2: 48.6 with one wave sharing 64-row tiles, against
+        // 49.9, loop 47.8).
+        if (tokens(2) && pairs >= 1792 && pairs < 2048) {
+            return kWave64;
+        }
+        return pairs < 2048 || !tokens(4) ? kBlock128 : kWave128;
+    }
+    // Prepared gates: 16-row tiles up to 128 pairs (128 x 2: 4.8, 32-row tiles 5.1,
+    // loop 5.9), 32-row tiles up to 256 (256 x 4: 8.4, 64-row tiles 8.6, loop 9.2;
+    // 256 x 16: 14.9, 16.9, loop 19.6)
+    if (pairs <= 128) {
+        return kBlock16;
+    }
+    const bool decay = a.gate_mode == KDA_GATE_DECAY;
+    // a pool of V-contiguous rows moves in 4-byte pieces, whole lines of them from the
+    // 32 rows of a tile; taller tiles touch them once per row (1024 x 2: 72 with
+    // 32-row tiles, 73 with 64-row, 131 with 128-row tiles, loop 79; 2048 x 8:
+    // 141, 149, 250, 261)
+    const bool vpool = decay && a.state_v_contiguous != 0;
+    // (decay gates' are five per CU: 320 x 4: 9.9, 64-row tiles 11.0, loop 12.0)
+    if (pairs <= (decay ? 320 : 256) || (vpool && tokens(8))) {
+        return kBlock32;
+    }
+    if (vpool) {
+        return kBlock64;
+    }
+    // 384 x 4: 64-row tiles 10.2, 32-row tiles 13.1, 128-row tiles 12.0, loop 11.9
+    // (decay gates 11.9, 14.8, 14.3, 13.0)
+    if (pairs <= 384) {
+        return kBlock64;
+    }
+    // 512 x 2: log gates 12.6 with 128-row tiles, 64-row tiles 15.0, loop 17.0; 512 x
+    // 8: 18.8, 16.4, 20.3; decay gates, 2: 16.9, 13.7, 17.8; 8: 22.3, 19.0, 21.1
+    if (pairs <= 512) {
+        return !decay && tokens(4) ? kBlock128 : kBlock64;
+    }
+    // 640 x 4: log gates 15.6 with 128-row tiles, 32-row tiles 18.6, loop 21.2;
+    // fp32 16.1, 20.2, 21.3; decay gates 20.4, 21.1, 23.7
+    if (pairs <= 768 && tokens(decay ? 4 : 6)) {
+        return kBlock128;
+    }
+    // Many pairs: 32-row tiles stream a few tokens' states best (2048 x 4: 48.3,
+    // 64-row tiles 50.8, 128-row tiles 52.8, loop 53.1; decay gates 55.6, 57.2, 60.4,
+    // 61.6; 8192 x 2: 177, 199, 191, 184); more tokens take the 64-row ones (16384 x
+    // 6: 396, 406; decay gates, 2048 x 16: 94, 99) and log gates past eight
+    // the 128-row ones (4096 x 16: 165, 64-row tiles 173, 32-row tiles 182)
+    if (tokens(5)) {
+        return kBlock32;
+    }
+    return !decay && !tokens(8) && tokens(16) ? kBlock128 : kBlock64;
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -1161,56 +1278,14 @@ extern "C" int kda_recurrent_launch_wide(const KdaRecurrentArgs *args, int32_t w
     if (kargs.head_count == 0 || kargs.head_begin + kargs.head_count > kargs.num_heads) {
         kargs.head_count = kargs.num_heads - kargs.head_begin;
     }
-    // Tile shape at D=128, by tokens per sequence and (sequence, head) pairs
-    // (measured on MI355X as graph replays, microseconds; "loop" is a token
-    // loop without shared blocks, which these shapes replaced).
-    // One token (decode): 32-lane rows, 2 rows per lane: 16-row tiles, eight
-    // workgroups per pair, which stream the state fastest (B=256, H=32: 173,
-    // against 182 with 32-row tiles); 8-row tiles below 128 pairs.
-    // Several tokens: blocks. Below 128 pairs 16-row tiles, whose eight
-    // workgroups per pair spread a short step over the CUs (2 x 4 tokens,
-    // H=32, checkpoints: 6.2, against 6.8 with 64-row tiles; loop 9.2). While
-    // all of them are resident at once (four workgroups of two per pair and
-    // CU, three with fp32 inputs' registers) 64-row tiles (16 x 20-120
-    // tokens, H=32: 115, against 147 with 128-row tiles; loop 253). Beyond,
-    // short sequences take 128-row tiles, which prepare a token once per pair
-    // and run in fewer rounds (48 x 4 tokens, H=16: 17.7 against 21.2; loop
-    // 27.2), long ones, bound by VALU issue, keep the 64-row tiles' higher
-    // occupancy (64 x 20-120 tokens, H=32: 399 against 414; loop 728). With
-    // 2048 pairs and more the state's traffic bounds a few tokens: up to four
-    // no barrier is worth its coupling of the waves' loads (one wave sharing,
-    // 512 x 4 tokens, H=32: 353, against 389; loop 383), up to six the 64-row
-    // tiles stream better (256 x 6, H=32, prepared gates: 191 against 196 and
-    // 215 with one wave sharing; loop 201).
-    // D=64: 64-row tiles are one workgroup per pair, 16-row tiles four (2 x
-    // 37-63 tokens, H=4: 17 against 25; 64 x 4, H=16: 14.9 against 9.1).
     const int64_t pairs = static_cast<int64_t>(a.num_seqs) * kargs.head_count;
-    const int64_t seqs = a.num_seqs;
-    const int64_t ntok = a.num_tokens;
-    Shape shape;
-    if (D == 128) {
-        const int64_t resident = a.qk_dtype == KDA_F32 ? 384 : 512;
-        if (ntok <= seqs) {
-            shape = pairs < 128 ? kDecode8 : kDecode16;
-        } else if (pairs < 128) {
-            shape = kBlock16;
-        } else if (pairs <= resident || ntok > 16 * seqs) {
-            shape = kBlock64;
-        } else if (pairs < 2048 || ntok > 6 * seqs) {
-            shape = kBlock128;
-        } else {
-            shape = ntok <= 4 * seqs ? kWave128 : kBlock64;
-        }
-    } else if (ntok <= seqs) {
-        shape = pairs >= 2048 ? kD64Large : kD64Small;
-    } else {
-        shape = pairs >= 256 ? kBlock64 : kBlock16;
-    }
+    const Shape shape = tile_shape(a, pairs);
     int rows_per_wg = 128;
     switch (shape) {
         case kDecode8: rows_per_wg = 8; break;
         case kDecode16: case kBlock16: case kD64Small: rows_per_wg = 16; break;
-        case kBlock64: case kD64Large: rows_per_wg = 64; break;
+        case kBlock32: rows_per_wg = 32; break;
+        case kBlock64: case kWave64: case kD64Large: rows_per_wg = 64; break;
         case kBlock128: case kWave128: break;
     }
     KernelFn fn = (D == 128) ? pick_kernel<128>(a.gate_mode, a.qk_dtype, a.v_dtype, shape)

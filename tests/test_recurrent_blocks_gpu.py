@@ -1,9 +1,9 @@
 """The recurrent kernel's token blocks against the oracle, at their edges.
 
 Several tokens per sequence run in blocks (16 tokens shared by a workgroup, or
-four by a wave); the launcher picks the tile by pairs (requests x heads),
-tokens per request and head dimension. Each case sits in one branch of that
-choice, with lengths on both sides of a block's end, empty requests, a padding
+four by a wave); the launcher picks the tile by gate form, pairs (requests x
+heads), tokens per request, head dimension and, for decay gates, pool layout.
+Each case sits in one branch of that choice, with lengths on both sides of a block's end, empty requests, a padding
 request, uncovered tokens and tracked prefixes; v is also passed from an
 address that no vector load may use. Tolerance: fp32 arithmetic on both sides
 (sums of 128 products, at most 40 steps of a decaying recurrence), 1e-5 of the
@@ -24,11 +24,13 @@ TOL = 1e-5
 # (heads, lengths, D): the branch that takes it
 BLOCK_CASES = {
     "tile16": (3, (0, 1, 2, 15, 16, 17, 33), 128),
-    "tile64": (16, (1, 3, 4, 5, 15, 16, 17, 0, 31, 32, 33, 2), 128),
+    "tile32": (16, (1, 3, 4, 5, 15, 16, 17, 0, 31, 32, 33, 2), 128),
+    "tile64": (32, (1, 3, 4, 5, 15, 16, 17, 0, 31, 32, 33, 2), 128),
     "tile128": (16, tuple([0, 1, 4, 5, 16, 17, 2, 3] * 5), 128),
     "tile64_many_long": (16, tuple([33, 16, 17, 40] * 9), 128),
     "wave": (64, tuple([0, 1, 2, 3, 4, 5, 8, 9] * 4), 128),
-    "tile64_many_short": (64, tuple([4, 5, 6, 7, 3, 5, 4, 6] * 4), 128),
+    "wave64": (64, tuple([0, 1, 2, 3, 4, 2, 1] * 4), 128),
+    "tile128_many_short": (64, tuple([4, 5, 6, 7, 3, 5, 4, 6] * 4), 128),
     "tile128_many": (64, tuple([0, 5, 8, 9, 16, 4, 17, 1] * 4), 128),
     "d64_tile16": (2, (1, 16, 17, 5, 0), 64),
     "d64_tile64": (16, tuple([1, 4, 16, 17] * 4), 64),
@@ -65,7 +67,8 @@ def test_raw_blocks(gpu_ops, name, aligned):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("heads,n,steps", [(4, 3, 4), (16, 16, 5), (16, 40, 17), (64, 32, 4), (64, 32, 6)])
+@pytest.mark.parametrize("heads,n,steps", [(4, 3, 4), (16, 16, 5), (16, 20, 3), (16, 30, 3), (16, 40, 4),
+                                           (16, 40, 17), (16, 64, 12), (64, 32, 4), (64, 32, 6)])
 def test_prepared_blocks_with_checkpoints(gpu_ops, heads, n, steps, dtype):
     lengths = [steps - (i % 3 if i % 4 == 1 else 0) for i in range(n)]
     D = 128
