@@ -19,6 +19,8 @@ namespace kda {
 // read the low words, which is what a conversion to int32 keeps. A caller with
 // int64 metadata then needs no conversion kernels before the launch (two of
 // about 4 us each: decode of 37 sequences, 32 heads, 33.0 -> 28.8 us).
+constexpr int32_t kWideAll =
+    KDA_WIDE_CU_SEQLENS | KDA_WIDE_STATE_INDICES | KDA_WIDE_TRACK_INDICES | KDA_WIDE_TRACK_LENS;
 template <class Args> struct Launch : Args {
     int32_t wide;
 

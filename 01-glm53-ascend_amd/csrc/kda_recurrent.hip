@@ -1224,7 +1224,7 @@ extern "C" int kda_recurrent_launch(const KdaRecurrentArgs *args, void *stream) 
 
 extern "C" int kda_recurrent_launch_wide(const KdaRecurrentArgs *args, int32_t wide, void *stream) {
     using namespace kda;
-    if (args == nullptr) {
+    if (args == nullptr || (wide & ~kWideAll) != 0) {
         return KDA_ERR_INVALID_ARGUMENT;
     }
     const KdaRecurrentArgs &a = *args;

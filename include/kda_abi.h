@@ -51,6 +51,8 @@
 extern "C" {
 #endif
 
+/* Raised when an existing entry point, structure or constant changes; entry points
+ * that are only added (the *_wide ones) leave it as it is. */
 #define KDA_ABI_VERSION 2
 
 typedef enum KdaStatus {
@@ -154,7 +156,8 @@ int kda_recurrent_launch(const KdaRecurrentArgs *args, void *stream);
 #define KDA_WIDE_TRACK_LENS 8
 
 /* kda_recurrent_launch with int64 metadata arrays: `wide` is a sum of KDA_WIDE_*
- * (0: all int32). No counterpart in the reference, which converts them first. */
+ * (0: all int32; other bits are KDA_ERR_INVALID_ARGUMENT). No counterpart in the
+ * reference, which converts them first. */
 int kda_recurrent_launch_wide(const KdaRecurrentArgs *args, int32_t wide, void *stream);
 
 typedef struct KdaChunkArgs {

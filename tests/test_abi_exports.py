@@ -237,3 +237,17 @@ def test_noalloc_rejects_what_its_scratch_cannot_hold(lib):
     assert b"noalloc" in lib.kda_status_string(5)
     a.head_dim = 64
     assert lib.kda_chunk_launch_noalloc(ctypes.byref(a), None) == 2  # unsupported, checked first
+
+
+def test_wide_launches_refuse_unknown_bits(lib):
+    """The int64 entry points take a sum of the four KDA_WIDE_* bits and nothing else."""
+    lib.kda_recurrent_launch_wide.restype = lib.kda_chunk_launch_wide.restype = ctypes.c_int
+    lib.kda_recurrent_launch_wide.argtypes = [ctypes.POINTER(_RecArgs), ctypes.c_int32, ctypes.c_void_p]
+    lib.kda_chunk_launch_wide.argtypes = [ctypes.POINTER(_ChunkArgs), ctypes.c_int32, ctypes.c_void_p,
+                                          ctypes.c_size_t, ctypes.c_void_p]
+    # no request: valid arguments return KDA_OK before any device call
+    rec = _RecArgs(num_heads=4, head_dim=128)
+    chunk = _ChunkArgs(num_heads=4, head_dim=128)
+    for wide, status in ((0, 0), (15, 0), (16, 1), (17, 1), (-1, 1), (1 << 30, 1)):
+        assert lib.kda_recurrent_launch_wide(ctypes.byref(rec), wide, None) == status, wide
+        assert lib.kda_chunk_launch_wide(ctypes.byref(chunk), wide, None, 0, None) == status, wide
