@@ -3701,7 +3701,7 @@ extern "C" int kda_chunk_launch(const KdaChunkArgs *args, void *workspace, size_
 extern "C" int kda_chunk_launch_wide(const KdaChunkArgs *args, int32_t wide, void *workspace,
                                      size_t workspace_bytes, void *stream) {
     using namespace kda::chunk;
-    if ((wide & ~kWideAll) != 0) {
+    if ((wide & ~kda::kWideAll) != 0) {
         return KDA_ERR_INVALID_ARGUMENT;
     }
     const int rc = check_args(args);
