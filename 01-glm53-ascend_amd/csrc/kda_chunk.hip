@@ -662,10 +662,10 @@ __device__ __forceinline__ void invert_blocks(const float (&lt)[16], float (&acc
     asm("s_nop 1\n\t"
         KDA_F1(0) KDA_F2(1) KDA_F3(2) KDA_F4(3) KDA_F5(4) KDA_F6(5) KDA_F7(6) KDA_F8(7)
         KDA_F9(8) KDA_F10(9) KDA_F11(10) KDA_F12(11) KDA_F13(12) KDA_F14(13) KDA_F15(14)
-        : [a0] "+v"(acc[0]), [a1] "+v"(acc[1]), [a2] "+v"(acc[2]), [a3] "+v"(acc[3]), [a4] "+v"(acc[4]),
-          [a5] "+v"(acc[5]), [a6] "+v"(acc[6]), [a7] "+v"(acc[7]), [a8] "+v"(acc[8]), [a9] "+v"(acc[9]),
-          [a10] "+v"(acc[10]), [a11] "+v"(acc[11]), [a12] "+v"(acc[12]), [a13] "+v"(acc[13]), [a14] "+v"(acc[14]),
-          [a15] "+v"(acc[15])
+        : [a0] "+&v"(acc[0]), [a1] "+&v"(acc[1]), [a2] "+&v"(acc[2]), [a3] "+&v"(acc[3]), [a4] "+&v"(acc[4]),
+          [a5] "+&v"(acc[5]), [a6] "+&v"(acc[6]), [a7] "+&v"(acc[7]), [a8] "+&v"(acc[8]), [a9] "+&v"(acc[9]),
+          [a10] "+&v"(acc[10]), [a11] "+&v"(acc[11]), [a12] "+&v"(acc[12]), [a13] "+&v"(acc[13]), [a14] "+&v"(acc[14]),
+          [a15] "+&v"(acc[15])
         : [l1] "v"(lt[1]), [l2] "v"(lt[2]), [l3] "v"(lt[3]), [l4] "v"(lt[4]), [l5] "v"(lt[5]), [l6] "v"(lt[6]),
           [l7] "v"(lt[7]), [l8] "v"(lt[8]), [l9] "v"(lt[9]), [l10] "v"(lt[10]), [l11] "v"(lt[11]),
           [l12] "v"(lt[12]), [l13] "v"(lt[13]), [l14] "v"(lt[14]), [l15] "v"(lt[15]));
