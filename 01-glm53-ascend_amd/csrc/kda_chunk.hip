@@ -791,9 +791,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const uint16_t *qp = static_cast<const uint16_t *>(a.q);
 
     // S3 work units: (row block I, channel half sh = slices 2sh and 2sh+1),
-    // each with its pairs (I, J <= I); the two halves of every product are
-    // summed through LDS (half 1 stores, half 0 adds after a barrier). Five
-    // half-pairs and two half-blocks per wave:  wave 0: (3,0) (0,0)   wave 1: (3,1) (0,1)
+    // each with its pairs (I, J <= I); the two halves of every product meet
+    // through LDS (each wave leaves half of its tiles to the other half's wave
+    // and sums the rest). Five half-pairs and two half-blocks per wave, (I, sh):
+    //        wave 0: (3,0) (0,0)   wave 1: (3,1) (0,1)
     //        wave 2: (2,0) (1,0)   wave 3: (2,1) (1,1)
     const int sh = wave & 1;
     const int IA = wave < 2 ? 3 : 2;
@@ -1018,7 +1019,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     };
 
     // The exact form of pair (I, J) over this wave's channel half, for a
-    // chunk whose anchor factors would be clamped: every element's own
+    // chunk whose anchor factors leave fp32's range: every element's own
     // e^(G_i - G_j) (<= 1 for j <= i under decay; the entries above the
     // diagonal, which nothing reads, are clamped), in fp32. For each row x
     // of the block, lane (r, gq) sums its 16 channels of Akk[16I + x][16J + r]
@@ -1062,8 +1063,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
     // ---- S3: Akk (-> L^T), Aqk (-> LT's lower triangle), q e^G fragments ----
     // Each wave sums its pairs over its channel half; the partial products
-    // stay in registers until the k and cumsum tiles are dead (after S4), and
-    // the halves are then summed in LT.
+    // stay in registers until the k and cumsum tiles are dead (after S4); then
+    // the halves exchange theirs through `part` and write the sums to LT.
     f32x4 pk[2][4], pq[2][4];  // this half's partials of pair (I, J): Akk, Aqk
     float *sc = reinterpret_cast<float *>(rec + kOffSc);
     bf16x8 Rh[2][2], Rl[2][2], Qh[2][2], Ql[2][2];
@@ -1116,10 +1117,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
     }
     // Each tile and half has scales of its own, from its largest values: a bound
-    // over the chunk (max |k|, max |q|, the largest step of a growing decay) is cheaper, but a
-    // row far below it, or after one growing token every row, loses its bits.
-    // Both blocks' four groups share one reduction (K1 of 8192 tokens, 32
-    // heads: 121 us, with a reduction for each group 126, with bounds 123).
+    // over the chunk (max |k|, max |q|, the largest step of a growing decay) is
+    // cheaper, but a row far below it, or after one growing token every row,
+    // loses its bits.
+    // Both blocks' four groups share one reduction (8192 tokens, 32 heads in all:
+    // 266 us, with a reduction for each pair of groups 269, with bounds 263).
     int qsh[2], ksh[2];
     wave_shifts(max_mag(qg[0]), max_mag(ke[0]), max_mag(qg[1]), max_mag(ke[1]), qsh[0], ksh[0], qsh[1], ksh[1]);
 #pragma unroll
@@ -1281,11 +1283,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             }
         }
     }
-    // A chunk beyond the anchors' span: S3's products were formed from
-    // clamped factors; the exact form replaces them here, behind S4 and
-    // before G and K die (the q rows reloaded, so nothing of S3 stays live
-    // for it). The flags are read only here: their wait would otherwise
-    // land on the cumsum's path.
+    // A chunk beyond the anchors' span: S3's factors may be infinite there and
+    // its products not finite, so every pair (I, J <= I) is formed again here,
+    // by the exact form, behind S4 and before G and K die (the q rows
+    // reloaded, so nothing of S3 stays live for it). The flags are read only
+    // here: their wait would otherwise land on the cumsum's path.
     const bool exact = __builtin_amdgcn_readfirstlane(sm.far[0] | sm.far[1] | sm.far[2] | sm.far[3]) != 0;
     if (__builtin_expect(exact, 0)) {  // laid out after the kernel's straight-line path
 #pragma unroll
@@ -3099,10 +3101,10 @@ __global__ __launch_bounds__(kAffThreads) void chunk_affine_combine_kernel(const
     }
 }
 
-// Chunks per correction workgroup (they share the staged S_s).
 constexpr int kAffCorrectThreads = 512;
 
-// One workgroup per (later segment s, head, `per` of the segment's chunks): o_t = bf16(o'_t + O_t S_s). S_s is staged once as bf16
+// One workgroup per (later segment s, head, `per` of the segment's chunks, which
+// share the staged S_s): o_t = bf16(o'_t + O_t S_s). S_s is staged once as bf16
 // hi + lo B fragments (64 KiB), each 16-row tile of O is split likewise, and
 // the product takes three passes (hi hi, hi lo, lo hi: about 2^-16 relative
 // per term). Wave w takes token rows [16 (w % 4), + 16) of chunks w / 4,

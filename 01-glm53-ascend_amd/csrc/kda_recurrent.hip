@@ -18,7 +18,7 @@
 // owns E = D/L of its K elements as E/4 16-byte vectors at K offsets
 // 4*kc + 4*L*j, so every wave-wide 16-byte load covers whole 4*L-element
 // segments of its rows -- complete cache lines. A lane holds the same K
-// elements of NP consecutive rows. The two K-reductions per token
+// elements of NP rows. The two K-reductions per token
 // (prediction and readout) are group sums over the L lanes (DPP, plus one
 // ds_swizzle when L = 32), so the state tile lives in VGPRs from the first
 // load to the single in-place write-back: HBM sees each state byte exactly
@@ -72,9 +72,10 @@ template <> struct Raw4<float> {
 
 // NP values of one v row, RS elements apart, as loaded (widened at use, so
 // the load is not waited for until the value is needed). Consecutive values
-// (RS = 1; the host guarantees the segment is aligned to its size) arrive in
-// 16-byte or smaller vectors: bf16 pairs packed in words, fp32 as is. Spread
-// ones arrive one element per load.
+// (RS = 1) arrive in 16-byte or smaller vectors from addresses aligned for them
+// (load) and one element per load from others (load_each; the caller looks at the
+// alignment): bf16 pairs packed in words, fp32 as is. Spread ones always arrive one
+// element per load.
 template <typename T, int NP, int RS> struct RowIn;
 template <int NP, int RS> struct RowIn<uint16_t, NP, RS> {
     static constexpr int W = RS == 1 ? NP / 2 : NP;
@@ -155,12 +156,9 @@ template <int NP, int RS> struct RowIn<float, NP, RS> {
     __device__ __forceinline__ float get(int i) const { return x[i]; }
 };
 
-// NP output values of one row, RS elements apart, written by the row
-// group's lanes kc: consecutive ones as one vector by every lane (the same
-// bytes to the same address -- a store with no branch around it, so the
-// loop's wait for the next token's loads never has to cover a store that
-// may or may not have been issued: 8 tokens x 256 sequences, H=32, 245 ->
-// 230 us), spread ones value i by lane i.
+// NP output values of one row, RS elements apart: consecutive ones (RS = 1) this
+// lane's own, written as vectors to an address aligned for them; spread ones held
+// alike by the row group's lanes kc, value i written by lane i.
 template <typename T, int NP, int RS>
 __device__ __forceinline__ void store_row(T *p, const float (&x)[NP], int kc) {
     if constexpr (RS == 1) {

@@ -106,7 +106,7 @@ def test_decode_padding_slot_and_untouched(gpu_ops):
                          [(torch.int64, torch.int32), (torch.int32, torch.int64),
                           (torch.int64, torch.int64)])
 def test_index_dtype_does_not_change_result(gpu_ops, index_dtype, starts_dtype):
-    """int64 metadata is narrowed on the device, never misread (test_kda_index_dtypes.py)."""
+    """int64 metadata gives what its int32 form gives (test_kda_index_dtypes.py)."""
     case = C.raw_case(4, (257,), indices=[3], slots=6, seed=5)
     base_out, base_pool = _run_raw(gpu_ops, case, prefill=True)
     pool = C.to_dev(case.pool, DEV)
@@ -302,7 +302,7 @@ def test_prepared_recurrent_decay_form(gpu_ops, k_contiguous):
     assert torch.equal(half[2, 4:], pool_k[2, 4:])
     assert not torch.equal(half[2, :4], pool_k[2, :4])
     # Neither layout makes a pool-sized working copy: a pool of 256 slots
-    # (128 MiB) costs the call no more than its small index conversions.
+    # (128 MiB) costs the call next to no memory.
     big = (C.to_dev(C.native_pool(256, H, D, seed=15), DEV) if k_contiguous
            else C.native_pool(256, H, D, seed=15).contiguous().to(DEV))
     torch.cuda.synchronize()
@@ -427,16 +427,18 @@ _KDA_DTYPE = {torch.bfloat16: 0, torch.float32: 1}
 @pytest.mark.parametrize("shift", [0, 1], ids=["aligned", "misaligned"])
 @pytest.mark.parametrize("form", sorted(_FORMS))
 @pytest.mark.parametrize("lengths,heads", [((1,) * 128, 1), ((2,) * 8, 16), ((4,) * 8, 16),
-                                           ((1, 7, 3, 5, 2, 6, 4, 8), 16), ((3,) * 64, 16)],
-                         ids=["decode", "2tok", "4tok", "ragged", "3tok-1024pairs"])
+                                           ((1, 7, 3, 5, 2, 6, 4, 8), 16), ((3,) * 64, 16),
+                                           ((2,) * 12, 16), ((3,) * 22, 16), ((4,) * 40, 16)],
+                         ids=["decode", "2tok", "4tok", "ragged", "3tok-1024pairs",
+                              "2tok-192pairs", "3tok-352pairs", "4tok-640pairs"])
 def test_tile_shapes_and_io_forms(gpu_ops, lengths, heads, form, shift):
-    """Every tile shape the launcher picks for D=128 with at least 128
-    (sequence, head) pairs (one token: 32-lane rows, 16-row tiles; two
-    tokens per sequence: 32-lane rows, 32-row tiles; more: 16-lane rows,
-    64-row tiles, or 128-row tiles from 1024 pairs, whose v and o rows move
-    as vectors), in every prepared input form, with v and out aligned or
-    shifted by one element (the per-element path), through the C ABI,
-    against the oracle."""
+    """The tile shapes the launcher picks for prepared gates, D=128 and at least
+    128 (sequence, head) pairs: one token, 32-lane rows and 16-row tiles; several,
+    token blocks of 16-lane rows, in 16-row tiles at 128 pairs, 32-row ones at
+    192 and 1024, 64-row ones at 352 and 128-row ones at 640, whose v and o
+    rows (from 32-row tiles up) move as vectors. In every prepared input form,
+    with v and out aligned or shifted by one element (the per-element path),
+    through the C ABI, against the oracle."""
     from sgl_glm53_ascend_ops._load import abi_library_path
 
     mode, qk_dt, v_dt = _FORMS[form]
