@@ -414,8 +414,9 @@ __device__ __forceinline__ void store_frags_f16_exp(char *base, int off, int idx
 
 __device__ __forceinline__ void seq_bounds(const ChunkLaunch &a, int n, int &bos, int &eos) {
     const int T = a.num_tokens;
-    bos = a.cu(n);
-    eos = a.cu(n + 1);
+    const int2 ends = a.cu_pair(n);
+    bos = ends.x;
+    eos = ends.y;
     bos = bos < 0 ? 0 : (bos > T ? T : bos);
     eos = eos < bos ? bos : (eos > T ? T : eos);
 }
@@ -3710,7 +3711,7 @@ extern "C" int kda_chunk_launch_wide(const KdaChunkArgs *args, int32_t wide, voi
     if (rc != KDA_OK || args->num_seqs == 0) {
         return rc;
     }
-    const ChunkLaunch a{*args, wide};
+    const ChunkLaunch a{{wide}, *args};
     if (workspace == nullptr || !aligned(workspace, 256)) {
         return KDA_ERR_WORKSPACE;
     }
@@ -3748,7 +3749,7 @@ extern "C" int kda_chunk_launch_noalloc(const KdaChunkArgs *args, void *stream) 
     if (rc != KDA_OK || args->num_seqs == 0) {
         return rc;
     }
-    const ChunkLaunch a{*args, 0};
+    const ChunkLaunch a{{0}, *args};
     const int T = a.num_tokens;
     const int H = a.num_heads;
     const bool whole = layout(T, a.num_seqs, H).total <= KDA_NOALLOC_SCRATCH_BYTES;

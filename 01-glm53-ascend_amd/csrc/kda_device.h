@@ -14,29 +14,40 @@
 
 namespace kda {
 
+constexpr int32_t kWideAll =
+    KDA_WIDE_CU_SEQLENS | KDA_WIDE_STATE_INDICES | KDA_WIDE_TRACK_INDICES | KDA_WIDE_TRACK_LENS;
+
 // A launch's arguments (KdaRecurrentArgs or KdaChunkArgs) with the width of its
 // metadata arrays (KDA_WIDE_* bits): of an int64 array's entries the kernels
 // read the low words, which is what a conversion to int32 keeps. A caller with
 // int64 metadata then needs no conversion kernels before the launch (two of
-// about 4 us each: decode of 37 sequences, 32 heads, 33.0 -> 28.8 us).
-constexpr int32_t kWideAll =
-    KDA_WIDE_CU_SEQLENS | KDA_WIDE_STATE_INDICES | KDA_WIDE_TRACK_INDICES | KDA_WIDE_TRACK_LENS;
-template <class Args> struct Launch : Args {
+// about 4 us each: decode of 37 sequences, 32 heads, 33.0 -> 28.8 us). The width
+// stands first, in the line of the arguments that a kernel loads at its start.
+struct Width {
     int32_t wide;
-
-    __device__ __forceinline__ int cu(int n) const { return this->cu_seqlens[at(n, KDA_WIDE_CU_SEQLENS)]; }
+};
+template <class Args> struct Launch : Width, Args {
+    // cu_seqlens[n] and [n + 1]
+    __device__ __forceinline__ int2 cu_pair(int n) const {
+        const char *p = at(this->cu_seqlens, n, KDA_WIDE_CU_SEQLENS);
+        return make_int2(word(p), word(p + (4 << shift(KDA_WIDE_CU_SEQLENS))));
+    }
     __device__ __forceinline__ int slot_index(int n) const {
-        return this->state_indices[at(n, KDA_WIDE_STATE_INDICES)];
+        return word(at(this->state_indices, n, KDA_WIDE_STATE_INDICES));
     }
     __device__ __forceinline__ int track_index(int n) const {
-        return this->track_indices[at(n, KDA_WIDE_TRACK_INDICES)];
+        return word(at(this->track_indices, n, KDA_WIDE_TRACK_INDICES));
     }
-    __device__ __forceinline__ int track_length(int n) const { return this->track_lens[at(n, KDA_WIDE_TRACK_LENS)]; }
+    __device__ __forceinline__ int track_length(int n) const {
+        return word(at(this->track_lens, n, KDA_WIDE_TRACK_LENS));
+    }
 
   private:
-    __device__ __forceinline__ int64_t at(int n, int bit) const {
-        return static_cast<int64_t>(n) << ((wide & bit) != 0 ? 1 : 0);
+    __device__ __forceinline__ int shift(int bit) const { return (this->wide & bit) != 0 ? 1 : 0; }
+    __device__ __forceinline__ const char *at(const int32_t *p, int n, int bit) const {
+        return reinterpret_cast<const char *>(p) + (static_cast<uint64_t>(static_cast<uint32_t>(n)) << (2 + shift(bit)));
     }
+    static __device__ __forceinline__ int word(const char *p) { return *reinterpret_cast<const int32_t *>(p); }
 };
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
