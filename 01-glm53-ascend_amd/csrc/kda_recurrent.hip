@@ -1124,7 +1124,10 @@ KernelFn pick_kernel(int gate, int qk_dtype, int v_dtype, Shape shape) {
 //
 // One token (decode), D = 128: 32-lane rows, 2 rows per lane: 16-row tiles, eight
 // workgroups per pair, which stream the state fastest (256 x 1, H=32: 173,
-// against 182 with 32-row tiles); 8-row tiles below 128 pairs.
+// against 182 with 32-row tiles; 96 x 1, log gates: 4.4, against 5.6 with 8-row
+// tiles, raw 5.1 against 5.9); 8-row tiles below 48 pairs (16: 3.1 against 3.2; 48:
+// 3.9 against 3.8) and, on a pool of V-contiguous rows, below 128 (72: 8.7
+// against 9.0).
 //
 // Several tokens, D = 128. What a tile shares is the token's preparation: long with
 // raw gates (four exponentials and a reciprocal per channel, the norms), short with
@@ -1143,8 +1146,10 @@ Shape tile_shape(const KdaRecurrentArgs &a, int64_t pairs) {
         }
         return pairs >= 256 ? kBlock64 : kBlock16;
     }
+    // a pool of V-contiguous rows moves in 4-byte pieces
+    const bool vpool = a.gate_mode == KDA_GATE_DECAY && a.state_v_contiguous != 0;
     if (tokens(1)) {
-        return pairs < 128 ? kDecode8 : kDecode16;
+        return pairs < (vpool ? 128 : 48) ? kDecode8 : kDecode16;
     }
     if (a.gate_mode == KDA_GATE_RAW) {
         // few pairs: 16-row tiles spread a step over most CUs (32 x 4: 5.13, 32-row
@@ -1183,11 +1188,9 @@ Shape tile_shape(const KdaRecurrentArgs &a, int64_t pairs) {
         return kBlock16;
     }
     const bool decay = a.gate_mode == KDA_GATE_DECAY;
-    // a pool of V-contiguous rows moves in 4-byte pieces, whole lines of them from the
-    // 32 rows of a tile; taller tiles touch them once per row (1024 x 2: 72 with
-    // 32-row tiles, 73 with 64-row, 131 with 128-row tiles, loop 79; 2048 x 8:
-    // 141, 149, 250, 261)
-    const bool vpool = decay && a.state_v_contiguous != 0;
+    // V-contiguous rows: a tile of 32 takes whole lines, taller ones touch them
+    // once per row (1024 x 2: 72 with 32-row tiles, 73 with 64-row, 131 with 128-row
+    // tiles, loop 79; 2048 x 8: 141, 149, 250, 261)
     // (decay gates' are five per CU: 320 x 4: 9.9, 64-row tiles 11.0, loop 12.0)
     if (pairs <= (decay ? 320 : 256) || (vpool && tokens(8))) {
         return kBlock32;

@@ -97,12 +97,13 @@ def test_prepared_blocks_with_checkpoints(gpu_ops, heads, n, steps, dtype):
 
 @pytest.mark.parametrize("k_contiguous", [True, False])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("n,steps", [(32, 3), (64, 5), (75, 4), (100, 3), (160, 3), (300, 9), (512, 4)])
+@pytest.mark.parametrize("n,steps", [(11, 1), (12, 1), (20, 1), (40, 1), (32, 3), (64, 5), (75, 4), (100, 3), (160, 3),
+                                     (300, 9), (512, 4)])
 def test_decay_blocks(gpu_ops, n, steps, dtype, k_contiguous):
-    """``prepared_recurrent`` (four heads) over its tiles, on both pool layouts,
-    with ragged lengths, a padding request, uncovered tokens and tracked prefixes."""
+    """``prepared_recurrent`` (four heads) over its tiles and one-token shapes, on
+    both pool layouts, with ragged lengths, a padding request, uncovered tokens and tracked prefixes."""
     H, D = 4, 128
-    lengths = [steps - (i % 3 if i % 4 == 1 else 0) for i in range(n)]
+    lengths = [max(0, steps - (i % 3 if i % 4 == 1 else 0)) for i in range(n)]
     case = C.prepared_case(H, lengths, dtype=torch.float32, slots=2 * n + 1, seed=19)
     indices = case.indices.clone()
     indices[2] = 0
