@@ -1155,8 +1155,12 @@ Shape tile_shape(const KdaRecurrentArgs &a, int64_t pairs) {
         // few pairs: 16-row tiles spread a step over most CUs (32 x 4: 5.13, 32-row
         // tiles 5.15, loop 6.1), from 48 pairs 32-row tiles fill them with half the
         // preparations (48 x 2: 4.8 against 5.2; 256 x 2: 8.0 against 8.8 with
-        // 64-row tiles, loop 8.5; 256 x 20-120: 63 against 82, loop 170)
-        if (pairs <= 32) {
+        // 64-row tiles, loop 8.5; 256 x 20-120: 63 against 82, loop 170). Up to 64 pairs
+        // 32-row tiles are at most one workgroup per CU, and nothing then shares a CU
+        // with the longest sequence: past verify lengths, prompts of unlike lengths take
+        // 16-row tiles (36 x 20-120: 39-45 against 42-49, 64 x 4-40: 12.6-19.7 against
+        // 13.8-19.5), and prompts of one length pay for it (64 x 100: 44.8 against 42.6)
+        if (pairs <= 32 || (pairs <= 64 && !tokens(8))) {
             return kBlock16;
         }
         if (pairs <= 256) {

@@ -24,6 +24,7 @@ TOL = 1e-5
 # (heads, lengths, D): the branch that takes it
 BLOCK_CASES = {
     "tile16": (3, (0, 1, 2, 15, 16, 17, 33), 128),
+    "tile16_long": (8, (0, 1, 16, 40, 17, 33), 128),
     "tile32": (16, (1, 3, 4, 5, 15, 16, 17, 0, 31, 32, 33, 2), 128),
     "tile64": (32, (1, 3, 4, 5, 15, 16, 17, 0, 31, 32, 33, 2), 128),
     "tile128": (16, tuple([0, 1, 4, 5, 16, 17, 2, 3] * 5), 128),
