@@ -1,8 +1,7 @@
 """Benchmark of the KDA hot path on one MI355X: decode tok/s + state HBM GB/s, prefill tok/s.
 
-Workload (BASELINE.json ``configs[1]``, the configuration the metric is quoted
-on): varlen recurrent decode, one token for each of 256 sequences, H=32,
-K=V=128, bf16 q/k/v (q, k L2-normalized), fp32 per-channel log decay
+Workload (the configuration the metric is quoted on): varlen recurrent
+decode, one token for each of 256 sequences, H=32, K=V=128, bf16 q/k/v (q, k L2-normalized), fp32 per-channel log decay
 ``g = logsigmoid(randn)`` and ``beta = sigmoid(randn)``, fp32 state pool of 512
 slots (``randn*0.05``, K-contiguous), ``state_indices`` a seeded random
 permutation of 256 of the slots, updated in place. One *step* is one call of
@@ -11,8 +10,8 @@ sequences by one token in place). ``value`` = tokens/s = 256 / step time.
 
 Also reported in the same JSON line:
 
-* ``prefill`` -- the chunked prefill of ``configs[2]`` (T=8192, one sequence,
-  H=32, K=V=128, chunk 64);
+* ``prefill`` -- the chunked prefill (T=8192, one sequence, H=32,
+  K=V=128, chunk 64);
 * ``roofline`` -- the decode kernel: algorithmic bytes / HIP-event time per
   call on the launch stream; ``traffic`` is the HBM bytes per launch from the
   committed rocprofv3 counter summary, used only while the kernel source it was
@@ -26,7 +25,7 @@ Also reported in the same JSON line:
   H16/32/64 x B1/32/128, the five checkpointed verify shapes, recurrent
   prefill H4/H8, each validated against the oracle and timed;
 * ``cpu_baseline`` -- this repository's torch oracle of the reference CPU path
-  on the host cores over a bounded sample; the same leg is the checker that
+  on the host cores over a bounded sample; the same leg
   validates every timed workload before it is timed (``validated``). A failed
   validation makes the run exit non-zero.
 
@@ -433,7 +432,7 @@ def run_raw_decode(steps, warmup, min_settle, check):
 
 
 # ---------------------------------------------------------------------------
-# the CPU baseline leg: the oracle timed on the host, and as the checker
+# the CPU baseline leg: the oracle timed on the host, and as the reference of every check
 # ---------------------------------------------------------------------------
 
 
@@ -452,7 +451,7 @@ def cpu_decode(case, sample_n=64, budget_s=10.0):
     """The oracle's recurrent decode (the reference CPU path's loop structure,
     bench/kda_chunk/kda_python.py:253-307) on the first ``sample_n`` of the
     config-2 sequences, on the host cores. Returns the baseline figures and the
-    oracle's outputs and states (the checker's reference for those sequences):
+    oracle's outputs and states (the reference for those sequences):
     their slots are renumbered 1..sample_n in a compact pool (0 stays 0)."""
     from oracle import kda_ref as R
 
@@ -489,7 +488,7 @@ def cpu_prefill(case, sample_t=512, budget_s=12.0):
     """The oracle's chunked prefill (bench/kda_chunk/kda_python.py:41-188) on
     the first ``sample_t`` of the config-3 tokens, all heads, on the host
     cores. Returns the baseline figures, the oracle's output and its state
-    after the sample (the checker's reference for the same prefix)."""
+    after the sample (the reference for the same prefix)."""
     from oracle import kda_ref as R
 
     torch.set_num_threads(os.cpu_count() or 1)
@@ -763,7 +762,7 @@ def main():
                                                     initial_state_indices=idx, cu_seqlens=cu,
                                                     scale=case.scale)
             torch.cuda.synchronize()
-            _log("cpu baseline / checker: oracle decode on host cores")
+            _log("cpu baseline / oracle: decode on host cores")
             cpu, ref_out, ref_pool, sidx = cpu_decode(case)
             n = ref_out.shape[1]
             slots = case.indices[:n].tolist()
@@ -816,7 +815,7 @@ def main():
                 track_state_indices=torch.tensor([2], dtype=torch.int32, device="cuda"),
                 track_state_lens=torch.tensor([sample_t], dtype=torch.int32, device="cuda"))
             torch.cuda.synchronize()
-            _log("cpu baseline / checker: oracle chunked prefill on host cores")
+            _log("cpu baseline / oracle: chunked prefill on host cores")
             pf_cpu, ref_out, ref_state = cpu_prefill(case, sample_t)
             validated["prefill"] = _errs(out[:, :sample_t].cpu(), ref_out, pool[2].cpu(),
                                          ref_state)
